@@ -243,7 +243,7 @@ struct JobOf {
                         }
                     }
                 }
-                bool flatten = Access::FLATTENS && used == count && !ragged;
+                bool flatten = Access::FLATTENS && (Out::ROW_MAJOR || Out::IS_SPLIT) && used == count && !ragged;
                 if constexpr (Access::FLATTENS) {
                     for (size_t i = 0; i < used; ++i) {
                         const auto& v = job.plane[i].prog.view;
@@ -263,32 +263,21 @@ struct JobOf {
                             v.h = v.img_h = 1;
                         }
                     }
-                    bool vec = Access::template aligned<Job::K>(v);
                     const char* const ofirst = reinterpret_cast<const char*>(out.data) + i * out.z_stride;
-                    vec = vec && aligned_to(ofirst, out_chunk) && (v.h == 1 || out.pitch % out_chunk == 0);
-                    if constexpr (Out::IS_SPLIT) vec = vec && out.chan_stride % out_chunk == 0;
-                    // outputs larger than the caches are written with streaming stores
-                    const bool stream = static_cast<size_t>(v.w) * v.h * count * sizeof(typename Out::Pixel) >= STREAM_STORE_MIN_BYTES;
-                    job.plane[i].flags = (vec ? FLAG_VECTOR_IO : 0u) | (vec && stream ? FLAG_STREAM_STORES : 0u) | (ragged ? FLAG_WHOLE_BOX : 0u);
+                    const auto out_aligned = [&](size_t bytes) {
+                        bool at = aligned_to(ofirst, bytes) && (v.h == 1 || out.pitch % bytes == 0);
+                        if constexpr (Out::IS_SPLIT) at = at && out.chan_stride % bytes == 0;
+                        return at;
+                    };
+                    const bool groups = Access::groups(v);
+                    const bool vec = Access::template aligned<Job::K>(v) && out_aligned(out_chunk);
+                    // outputs larger than the caches are written with streaming stores, where rows start at whole dwords
+                    const bool stream = groups && out_aligned(4) && (Out::ROW_MAJOR || Out::IS_SPLIT) && static_cast<size_t>(v.w) * v.h * count * sizeof(typename Out::Pixel) >= STREAM_STORE_MIN_BYTES;
+                    job.plane[i].flags = (groups ? FLAG_GROUP_IO : 0u) | (vec ? FLAG_VECTOR_IO : 0u) | (stream ? FLAG_STREAM_STORES : 0u) | (ragged ? FLAG_WHOLE_BOX : 0u);
                     max_w = v.w > max_w ? v.w : max_w;
                     max_h = v.h > max_h ? v.h : max_h;
                 }
-                // thread columns per block: enough to span the widest row, at most the whole block
-                const unsigned groups = ceil_div(static_cast<unsigned>(max_w), Job::K);
-                unsigned shift = 0;
-                while ((1u << shift) < groups && shift < 8u) ++shift;
-                if (shift < 4u) shift = 4u; // keep a wave's accesses within a few rows
-                job.tx_shift = shift;
-                job.grid_x = ceil_div(groups, 1u << shift);
-                job.grid_y = ceil_div(static_cast<unsigned>(max_h), BLOCK_THREADS >> shift);
-                job.pair_limit = 0u;
-                if constexpr (N == 1 && Access::PAIRS_ROWS) {
-                    // one row per block row: rows that share a chroma row are handed to the same XCD
-                    if (shift == 8u) {
-                        const unsigned total = job.grid_x * job.grid_y, unit = 16u * job.grid_x; // whole turns of all XCDs, whole row pairs
-                        job.pair_limit = total / unit * unit;
-                    }
-                }
+                job.plan(ceil_div(static_cast<unsigned>(max_w), Job::K), ceil_div(static_cast<unsigned>(max_h), Job::ROWS));
                 return job;
             }
         } else {

@@ -105,63 +105,48 @@ __device__ __attribute__((always_inline)) inline void wave_sync() {
 }
 
 constexpr int gcd(int a, int b) { return b == 0 ? a : gcd(b, a % b); }
-// widest transaction (16, 8 or 4 bytes) that tiles NBYTES
+// widest power of two (at most 16 bytes) that divides NBYTES: the natural alignment of a run of NBYTES
 constexpr int chunk_bytes(int nbytes) { return gcd(nbytes, 16); }
 
-// NBYTES (a multiple of 4) from `p`, which is aligned to chunk_bytes(NBYTES)
+// NBYTES (a multiple of 4) from and to an address of any alignment, with the fewest wide accesses (dwordx4, x3, x2, one dword):
+// global memory takes them at every byte address, so rows that start anywhere, as the tight rows of an image of odd width do,
+// move with the same instructions as aligned ones.  (3254 x 1948 NV12 to float3: 38.2 us one sample at a time, 22.8 us this way.)
+// The loads are of vector type, not copies of bytes: of a copy the compiler drops the bytes that the chain does not use and
+// fetches the others one by one (a 16-byte group of uchar4 whose alpha is dropped became eight loads).
+typedef unsigned int dword_anywhere __attribute__((aligned(1)));
+typedef u32x2 u32x2_anywhere __attribute__((aligned(1)));
+typedef u32x4 u32x4_anywhere __attribute__((aligned(1)));
 template <int NBYTES>
 __device__ __attribute__((always_inline)) inline void load_words(const void* p, unsigned int* w) {
-    constexpr int C = chunk_bytes(NBYTES);
-    static_assert(NBYTES % 4 == 0 && C >= 4, "vector I/O moves whole dwords");
-    if constexpr (C == 16) {
+    static_assert(NBYTES % 4 == 0, "vector I/O moves whole dwords");
+    constexpr int FOURS = NBYTES / 16, REST = NBYTES / 4 - 4 * FOURS;
+    const char* const from = static_cast<const char*>(p);
 #pragma unroll
-        for (int i = 0; i < NBYTES / 16; ++i) {
-            const u32x4 v = static_cast<const u32x4*>(p)[i];
-            w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
-        }
-    } else if constexpr (C == 8) {
+    for (int i = 0; i < FOURS; ++i) {
+        const u32x4 v = reinterpret_cast<const u32x4_anywhere*>(from)[i];
+        w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
+    }
+    if constexpr (REST == 2) {
+        const u32x2 v = *reinterpret_cast<const u32x2_anywhere*>(from + 16 * FOURS);
+        w[4 * FOURS] = v.x; w[4 * FOURS + 1] = v.y;
+    } else { // (three neighbouring dwords are merged into one load)
 #pragma unroll
-        for (int i = 0; i < NBYTES / 8; ++i) {
-            const u32x2 v = static_cast<const u32x2*>(p)[i];
-            w[2 * i] = v.x; w[2 * i + 1] = v.y;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NBYTES / 4; ++i) w[i] = static_cast<const unsigned int*>(p)[i];
+        for (int i = 0; i < REST; ++i) w[4 * FOURS + i] = reinterpret_cast<const dword_anywhere*>(from + 16 * FOURS)[i];
     }
 }
+__device__ __attribute__((always_inline)) inline u32x4 load_piece(const char* p) { return *reinterpret_cast<const u32x4_anywhere*>(p); }
+__device__ __attribute__((always_inline)) inline void store_piece(char* p, const u32x4& v) { *reinterpret_cast<u32x4_anywhere*>(p) = v; }
 // STREAM: non-temporal stores.  Only for accesses where a wave writes whole cache lines (consecutive lanes,
-// consecutive 16/8/4-byte pieces): they then leave the caches alone and measurably raise the write bandwidth;
-// on partial lines they are a pessimisation.
-template <bool STREAM, typename V>
-__device__ __attribute__((always_inline)) inline void store_piece(V* p, const V& v) {
-    if constexpr (STREAM) {
-        __builtin_nontemporal_store(v, p);
-    } else {
-        *p = v;
-    }
-}
+// consecutive pieces): they then leave the caches alone and measurably raise the write bandwidth; on partial lines they
+// are a pessimisation.
 template <int NBYTES, bool STREAM = false>
 __device__ __attribute__((always_inline)) inline void store_words(void* p, const unsigned int* w) {
-    constexpr int C = chunk_bytes(NBYTES);
-    static_assert(NBYTES % 4 == 0 && C >= 4, "vector I/O moves whole dwords");
-    if constexpr (C == 16) {
+    static_assert(NBYTES % 4 == 0, "vector I/O moves whole dwords");
+    if constexpr (STREAM) {
 #pragma unroll
-        for (int i = 0; i < NBYTES / 16; ++i) {
-            u32x4 v;
-            v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
-            store_piece<STREAM>(static_cast<u32x4*>(p) + i, v);
-        }
-    } else if constexpr (C == 8) {
-#pragma unroll
-        for (int i = 0; i < NBYTES / 8; ++i) {
-            u32x2 v;
-            v.x = w[2 * i]; v.y = w[2 * i + 1];
-            store_piece<STREAM>(static_cast<u32x2*>(p) + i, v);
-        }
+        for (int i = 0; i < NBYTES / 4; ++i) __builtin_nontemporal_store(w[i], static_cast<dword_anywhere*>(p) + i); // (merged into wide stores)
     } else {
-#pragma unroll
-        for (int i = 0; i < NBYTES / 4; ++i) store_piece<STREAM>(static_cast<unsigned int*>(p) + i, w[i]);
+        __builtin_memcpy(p, w, NBYTES);
     }
 }
 
@@ -284,7 +269,24 @@ __device__ __attribute__((always_inline)) inline void pack_pixels(const O* v, un
     }
 }
 
-// K consecutive pixels starting at x0 (caller guarantees the alignment that chunk_bytes asks for)
+// and back: element i of the dwords of a run, by shifts (through a copy of bytes the elements would take their way through memory)
+template <typename B>
+__device__ __attribute__((always_inline)) inline B element_of(const unsigned int* w, const int i) {
+    static_assert(sizeof(B) <= 2, "elements of one or two bytes");
+    constexpr int PER = 4 / static_cast<int>(sizeof(B));
+    using U = std::conditional_t<sizeof(B) == 1, unsigned char, unsigned short>;
+    return static_cast<B>(static_cast<U>(w[i / PER] >> (8 * static_cast<int>(sizeof(B)) * (i % PER))));
+}
+// ... and put there, into dwords that hold zeros
+template <typename B>
+__device__ __attribute__((always_inline)) inline void put_element(unsigned int* w, const int i, const B v) {
+    static_assert(sizeof(B) <= 2, "elements of one or two bytes");
+    constexpr int PER = 4 / static_cast<int>(sizeof(B));
+    using U = std::conditional_t<sizeof(B) == 1, unsigned char, unsigned short>;
+    w[i / PER] |= static_cast<unsigned int>(static_cast<U>(v)) << (8 * static_cast<int>(sizeof(B)) * (i % PER));
+}
+
+// K consecutive pixels starting at x0
 template <int K, bool STREAM = false, typename O>
 __device__ __attribute__((always_inline)) inline void store_group(const PackedOut<O>& out, int x0, int y, int z, const O* v) {
     constexpr int NB = K * static_cast<int>(sizeof(O));
@@ -292,7 +294,7 @@ __device__ __attribute__((always_inline)) inline void store_group(const PackedOu
     pack_pixels<K>(v, w);
     char* const row = reinterpret_cast<char*>(out.data) + static_cast<size_t>(z) * out.z_stride + static_cast<size_t>(y) * out.pitch;
     // a thread's K pixels are one transaction only when they fill exactly one piece
-    store_words<NB, STREAM && NB == chunk_bytes(NB)>(row + static_cast<size_t>(x0) * sizeof(O), w);
+    store_words<NB, STREAM && NB <= 16>(row + static_cast<size_t>(x0) * sizeof(O), w);
 }
 template <int K, bool STREAM = false, typename O>
 __device__ __attribute__((always_inline)) inline void store_group(const SplitOut<O>& out, int x0, int y, int z, const O* v) {
@@ -306,7 +308,54 @@ __device__ __attribute__((always_inline)) inline void store_group(const SplitOut
         for (int k = 0; k < K; ++k) ch[k] = vectorAt(c, v[k]);
         unsigned int w[NB / 4];
         pack_elements<K>(ch, w);
-        store_words<NB, STREAM && NB == chunk_bytes(NB)>(row + c * out.chan_stride + static_cast<size_t>(x0) * sizeof(B), w);
+        store_words<NB, STREAM && NB <= 16>(row + c * out.chan_stride + static_cast<size_t>(x0) * sizeof(B), w);
+    }
+}
+// {Y, U, V} pixels into a raw YUV image.  One pixel: WriteYUV's own rule for which pixel writes a chroma sample.
+template <PixelFormat PF>
+__device__ __attribute__((always_inline)) inline void store_one(const YuvOut<PF>& out, int x, int y, int, const typename YuvOut<PF>::Pixel& v) {
+    using Base = typename YuvOut<PF>::Base;
+    const RawImage<PF> raw{ RawPtr<ND::_2D, Base>{ out.data, PtrDims<ND::_2D>(0u, 0u, out.pitch) }, out.img_w, out.img_h };
+    WriteYUV<PF>::exec(Point(x, y), v, raw);
+}
+// K consecutive pixels from an even x0 on: their luma samples, and the chroma pairs of the pixels that write them (the even
+// ones; in NV21 the odd ones of odd rows).  K samples of each are one store.
+template <int K, bool STREAM = false, PixelFormat PF>
+__device__ __attribute__((always_inline)) inline void store_group(const YuvOut<PF>& out, int x0, int y, int, const typename YuvOut<PF>::Pixel* v) {
+    using Base = typename YuvOut<PF>::Base;
+    using Layout = fk::detail::YuvLayout<PF>;
+    static_assert(K % 2 == 0 && K * sizeof(Base) % 4 == 0, "whole chroma pairs, whole dwords");
+    char* const base = reinterpret_cast<char*>(out.data);
+    if constexpr (Layout::semi_planar) {
+        constexpr int NB = K * static_cast<int>(sizeof(Base));
+        constexpr int PICK = PF == PixelFormat::NV21 ? 1 : 0; // the pixel of a pair, and the row of a row pair, that writes the chroma
+        Base e[K];
+        unsigned int w[NB / 4];
+#pragma unroll
+        for (int k = 0; k < K; ++k) e[k] = v[k].x;
+        pack_elements<K>(e, w);
+        store_words<NB, STREAM>(base + static_cast<size_t>(y) * out.pitch + static_cast<size_t>(x0) * sizeof(Base), w);
+        if (Layout::row_shift == 1 && (y & 1) != PICK) return;
+#pragma unroll
+        for (int k = 0; k < K; k += 2) {
+            e[k + Layout::u] = v[k + PICK].y;
+            e[k + Layout::v] = v[k + PICK].z;
+        }
+        pack_elements<K>(e, w);
+        store_words<NB, STREAM>(base + (static_cast<size_t>(out.img_h) + (y >> Layout::row_shift)) * out.pitch + static_cast<size_t>(x0) * sizeof(Base), w);
+    } else {
+        constexpr int NB = 2 * K * static_cast<int>(sizeof(Base));
+        Base e[2 * K];
+        unsigned int w[NB / 4];
+#pragma unroll
+        for (int k = 0; k < K; k += 2) {
+            e[2 * k + Layout::y0] = v[k].x;
+            e[2 * k + Layout::y1] = v[k + 1].x;
+            e[2 * k + Layout::u] = v[k].y;
+            e[2 * k + Layout::v] = v[k].z;
+        }
+        pack_elements<2 * K>(e, w);
+        store_words<NB, STREAM>(base + static_cast<size_t>(y) * out.pitch + 2 * static_cast<size_t>(x0) * sizeof(Base), w);
     }
 }
 // One or the other, chosen at run time (block-uniform).  The empty asm keeps the compiler from merging the two stores
@@ -336,22 +385,25 @@ __device__ __attribute__((always_inline)) inline unsigned int pack3(const P& p) 
 }
 } // namespace dev
 
-// Pixels per thread: the smallest power of two that makes the wider side a whole number of 16-byte transactions and
-// the narrower side a whole number of dwords.
+// Pixels per thread: the smallest power of two that makes the wider side one 12-byte access or whole 16-byte ones, and the
+// narrower side whole dwords.  Small counts leave more waves to a launch (with 16 three-byte pixels per thread a 4K frame was one
+// round of waves, nothing overlapping their loads with other waves' stores: 8.7 us; with one 12-byte store per row and thread 7.7 us);
+// 12-byte pixels take four, whose 48 bytes are re-arranged into 16-byte accesses through LDS.
 template <typename S, typename O, bool SPLIT>
 constexpr int pixels_per_thread() {
     const int ss = static_cast<int>(sizeof(S));
     const int so = SPLIT ? static_cast<int>(sizeof(VBase<O>)) : static_cast<int>(sizeof(O));
     const int big = ss > so ? ss : so, small = ss > so ? so : ss;
     for (int k = 1; k <= 16; k *= 2) {
-        if ((k * big) % 16 == 0 && (k * small) % 4 == 0) return k;
+        if (((k * big == 12 && big < 12) || (k * big) % 16 == 0) && (k * small) % 4 == 0) return k;
     }
     return 16;
 }
 
 // ---- source access -----------------------------------------------------------------------------------------------
-// SourceAccess<View>: one pixel of the window (load_one), K consecutive pixels of a row with vector loads (load_group,
-// when the host found the alignment that needs: `aligned`), and the pixels per thread that suit an output pixel type.
+// SourceAccess<View>: one pixel of the window (load_one), K consecutive pixels of a row with vector loads (load_group, at any
+// byte alignment; `groups` says whether the window's pixels form such groups: whole chroma pairs, `aligned` whether they lie at natural alignment),
+// and the pixels per thread that suit an output pixel type.
 template <typename View>
 struct SourceAccess;
 
@@ -359,7 +411,7 @@ template <typename T>
 struct SourceAccess<PlainView<T>> {
     using View = PlainView<T>;
     static constexpr bool FLATTENS = true; // contiguous rows may be treated as one long row
-    static constexpr bool PAIRS_ROWS = false;
+    static constexpr int ROWS = 1;
     template <typename O, bool SPLIT>
     static constexpr int pixels() { return pixels_per_thread<T, O, SPLIT>(); }
     template <int K>
@@ -370,13 +422,61 @@ struct SourceAccess<PlainView<T>> {
     __device__ __attribute__((always_inline)) static inline T load_one(const View& v, int x, int y) {
         return fk::detail::read_element(reinterpret_cast<const T*>(row(v, y)) + x);
     }
-    template <int K>
-    __device__ __attribute__((always_inline)) static inline void load_group(const View& v, int x0, int y, T* out) {
-        constexpr int NB = K * static_cast<int>(sizeof(T));
-        unsigned int w[NB / 4];
-        dev::load_words<NB>(row(v, y) + static_cast<size_t>(x0) * sizeof(T), w);
-        __builtin_memcpy(out, w, NB);
+    __device__ __attribute__((always_inline)) static inline T one_channel(const VBase<T> e) {
+        if constexpr (validCUDAVec<T>) return T{ e };
+        else return e;
     }
+    // K pixels as the dwords they occupy.  They stay dwords until a pixel is taken out of them: an array of small pixels that is
+    // filled on two paths (whole groups, cut groups) ends up in memory.
+    template <int K>
+    struct Group {
+        unsigned int w[K * sizeof(T) / 4];
+        __device__ __attribute__((always_inline)) inline T pixel(const int k) const {
+            using B = VBase<T>;
+            if constexpr (sizeof(B) <= 2) {
+                if constexpr (cn<T> == 1) return one_channel(dev::element_of<B>(w, k));
+                else if constexpr (cn<T> == 2) return T{ dev::element_of<B>(w, 2 * k), dev::element_of<B>(w, 2 * k + 1) };
+                else if constexpr (cn<T> == 3) return T{ dev::element_of<B>(w, 3 * k), dev::element_of<B>(w, 3 * k + 1), dev::element_of<B>(w, 3 * k + 2) };
+                else return T{ dev::element_of<B>(w, 4 * k), dev::element_of<B>(w, 4 * k + 1), dev::element_of<B>(w, 4 * k + 2), dev::element_of<B>(w, 4 * k + 3) };
+            } else {
+                T p;
+                __builtin_memcpy(&p, w + k * (sizeof(T) / 4), sizeof(T));
+                return p;
+            }
+        }
+        __device__ __attribute__((always_inline)) inline void put(const int k, const T& p) { // (into a group of zeros)
+            using B = VBase<T>;
+            if constexpr (sizeof(B) <= 2) {
+#pragma unroll
+                for (int c = 0; c < cn<T>; ++c) dev::put_element<B>(w, cn<T> * k + c, vectorAt(c, p));
+            } else {
+                __builtin_memcpy(w + k * (sizeof(T) / 4), &p, sizeof(T));
+            }
+        }
+    };
+    template <int K>
+    __device__ __attribute__((always_inline)) static inline void load_group(const View& v, int x0, int y, Group<K>& out) {
+        dev::load_words<K * static_cast<int>(sizeof(T))>(row(v, y) + static_cast<size_t>(x0) * sizeof(T), out.w);
+    }
+    // The same pixel by pixel, for a group that is not whole: without a branch between the loads, columns past the row's end
+    // repeat its last pixel (and are not stored); pixels outside the parent image (WHOLE_BOX) are zero.
+    template <int K>
+    __device__ __attribute__((always_inline)) static inline void load_each(const View& v, const bool whole_box, int x0, int y, Group<K>& out) {
+        T p[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int x = x0 + k < v.w ? x0 + k : v.w - 1;
+            const bool in_parent = !whole_box || (v.oy + y < v.img_h && v.ox + x < v.img_w);
+            p[k] = load_one(v, in_parent ? x : -v.ox, in_parent ? y : -v.oy);
+        }
+        __builtin_memset(out.w, 0, sizeof(out.w));
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int x = x0 + k < v.w ? x0 + k : v.w - 1;
+            if (!whole_box || (v.oy + y < v.img_h && v.ox + x < v.img_w)) out.put(k, p[k]);
+        }
+    }
+    static bool groups(const View&) { return true; }
     template <int K>
     static bool aligned(const View& v) {
         constexpr size_t chunk = dev::chunk_bytes(K * static_cast<int>(sizeof(T)));
@@ -429,13 +529,15 @@ struct SourceAccess<YuvView<PF>> {
         if constexpr (Layout::semi_planar) return Layout::row_shift == 1;
         else return false;
     }
-    static constexpr bool PAIRS_ROWS = pairs_rows();
-    // smallest power of two >= 4 whose output run is whole 16-byte pieces and whose luma run is whole dwords
+    // Rows per thread: a thread of a 4:2:0 format takes a row pair, so that its chroma samples are read once and what is
+    // computed from them alone is computed once for the four pixels that share them.
+    static constexpr int ROWS = pairs_rows() ? 2 : 1;
+    // pixels_per_thread's rule over the output run and the luma run, for whole chroma pairs
     template <typename O, bool SPLIT>
     static constexpr int pixels() {
         const int so = SPLIT ? static_cast<int>(sizeof(VBase<O>)) : static_cast<int>(sizeof(O));
-        for (int k = 4; k <= 16; k *= 2) {
-            if ((k * so) % 16 == 0 && (k * static_cast<int>(sizeof(Base))) % 4 == 0) return k;
+        for (int k = 2; k <= 16; k *= 2) {
+            if (((k * so == 12 && so < 12) || (k * so) % 16 == 0) && (k * static_cast<int>(sizeof(Base))) % 4 == 0) return k;
         }
         return 16;
     }
@@ -447,33 +549,78 @@ struct SourceAccess<YuvView<PF>> {
                                 static_cast<uint>(v.img_h) };
         return ReadYUV<PF>::exec(Point(v.ox + x, v.oy + y), raw);
     }
+    // K pixels as the dwords they lie in: the luma run and the run of chroma pairs that covers it (semi-planar), or one run of
+    // 4:2:2 samples
+    template <int K>
+    struct Group {
+        static constexpr int ND = group_bytes<K>() / 4;
+        unsigned int w[ND], c[Layout::semi_planar ? ND : 1];
+        __device__ __attribute__((always_inline)) inline Pixel pixel(const int k) const {
+            const int pair = k & ~1;
+            if constexpr (Layout::semi_planar) return Pixel{ dev::element_of<Base>(w, k), dev::element_of<Base>(c, pair + Layout::u), dev::element_of<Base>(c, pair + Layout::v) };
+            else return Pixel{ dev::element_of<Base>(w, 2 * pair + ((k & 1) ? Layout::y1 : Layout::y0)), dev::element_of<Base>(w, 2 * pair + Layout::u), dev::element_of<Base>(w, 2 * pair + Layout::v) };
+        }
+    };
+    __device__ __attribute__((always_inline)) static inline const char* run(const View& v, const size_t row, int x) {
+        return reinterpret_cast<const char*>(v.data) + row * v.pitch + static_cast<size_t>(v.ox + x) * ((Layout::semi_planar ? 1 : 2) * sizeof(Base));
+    }
+    static constexpr int chroma_shift() {
+        if constexpr (Layout::semi_planar) return Layout::row_shift;
+        else return 0;
+    }
+    __device__ __attribute__((always_inline)) static inline size_t chroma_row(const View& v, int y) { return static_cast<size_t>(v.img_h) + ((v.oy + y) >> chroma_shift()); }
     // x0 and v.ox are even: the K pixels are K/2 whole chroma pairs
     template <int K>
-    __device__ __attribute__((always_inline)) static inline void load_group(const View& v, int x0, int y, Pixel* out) {
-        const int px = v.ox + x0, py = v.oy + y;
-        constexpr int NB = group_bytes<K>();
-        if constexpr (Layout::semi_planar) {
-            const char* const base = reinterpret_cast<const char*>(v.data);
-            unsigned int wl[NB / 4], wc[NB / 4];
-            dev::load_words<NB>(base + static_cast<size_t>(py) * v.pitch + static_cast<size_t>(px) * sizeof(Base), wl);
-            dev::load_words<NB>(base + (static_cast<size_t>(v.img_h) + (py >> Layout::row_shift)) * v.pitch + static_cast<size_t>(px) * sizeof(Base), wc);
-            Base luma[K], chroma[K];
-            __builtin_memcpy(luma, wl, NB);
-            __builtin_memcpy(chroma, wc, NB);
+    __device__ __attribute__((always_inline)) static inline void load_group(const View& v, int x0, int y, Group<K>& out) {
+        dev::load_words<group_bytes<K>()>(run(v, static_cast<size_t>(v.oy + y), x0), out.w);
+        if constexpr (Layout::semi_planar) dev::load_words<group_bytes<K>()>(run(v, chroma_row(v, y), x0), out.c);
+    }
+    // the same of rows y and y_below (y + 1, or y again) of a 4:2:0 image, which share their chroma: row v.oy + y of the image is even
+    template <int K>
+    __device__ __attribute__((always_inline)) static inline void load_group_pair(const View& v, int x0, int y, int y_below, Group<K>& upper, Group<K>& lower) {
+        load_group<K>(v, x0, y, upper);
+        dev::load_words<group_bytes<K>()>(run(v, static_cast<size_t>(v.oy + y_below), x0), lower.w);
 #pragma unroll
-            for (int k = 0; k < K; ++k) out[k] = Pixel{ luma[k], chroma[(k & ~1) + Layout::u], chroma[(k & ~1) + Layout::v] };
-        } else {
-            unsigned int w[NB / 4];
-            dev::load_words<NB>(reinterpret_cast<const char*>(v.data) + static_cast<size_t>(py) * v.pitch + 2 * static_cast<size_t>(px) * sizeof(Base), w);
-            Base quad[2 * K];
-            __builtin_memcpy(quad, w, NB);
+        for (int i = 0; i < Group<K>::ND; ++i) lower.c[i] = upper.c[i];
+    }
+    // sample by sample, for a group (from an even v.ox + x0 on) that the window cuts: columns past its end repeat its last pixel
+    template <int K>
+    __device__ __attribute__((always_inline)) static inline void load_each(const View& v, const bool, int x0, int y, Group<K>& out) {
+        __builtin_memset(out.w, 0, sizeof(out.w));
+        __builtin_memset(out.c, 0, sizeof(out.c));
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const int q = 4 * (k >> 1);
-                out[k] = Pixel{ quad[q + ((k & 1) ? Layout::y1 : Layout::y0)], quad[q + Layout::u], quad[q + Layout::v] };
+        for (int k = 0; k < K; ++k) {
+            const int x = x0 + k < v.w ? x0 + k : v.w - 1;
+            const Pixel p = load_one(v, x, y);
+            const int pair = k & ~1;
+            if constexpr (Layout::semi_planar) {
+                dev::put_element<Base>(out.w, k, p.x);
+                if (k == pair) {
+                    dev::put_element<Base>(out.c, pair + Layout::u, p.y);
+                    dev::put_element<Base>(out.c, pair + Layout::v, p.z);
+                }
+            } else {
+                dev::put_element<Base>(out.w, 2 * pair + ((k & 1) ? Layout::y1 : Layout::y0), p.x);
+                if (k == pair) {
+                    dev::put_element<Base>(out.w, 2 * pair + Layout::u, p.y);
+                    dev::put_element<Base>(out.w, 2 * pair + Layout::v, p.z);
+                }
             }
         }
     }
+    template <int K>
+    __device__ __attribute__((always_inline)) static inline void load_each_pair(const View& v, int x0, int y, int y_below, Group<K>& upper, Group<K>& lower) {
+        load_each<K>(v, false, x0, y, upper);
+        __builtin_memset(lower.w, 0, sizeof(lower.w));
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int x = x0 + k < v.w ? x0 + k : v.w - 1;
+            dev::put_element<Base>(lower.w, k, fk::detail::yuv_row(v.data, v.pitch, static_cast<size_t>(v.oy + y_below))[v.ox + x]);
+        }
+#pragma unroll
+        for (int i = 0; i < Group<K>::ND; ++i) lower.c[i] = upper.c[i];
+    }
+    static bool groups(const View& v) { return (v.ox & 1) == 0; }
     template <int K>
     static bool aligned(const View& v) {
         constexpr size_t chunk = dev::chunk_bytes(group_bytes<K>());
@@ -570,7 +717,9 @@ __device__ __attribute__((always_inline)) inline void fill_default(const Out& ou
 } // namespace dev
 
 // ---- pointwise ---------------------------------------------------------------------------------------------------
-enum : unsigned { FLAG_VECTOR_IO = 1u, FLAG_STREAM_STORES = 2u, FLAG_SOURCE_TILE = 4u, FLAG_WHOLE_BOX = 8u, FLAG_PACKED_TILE = 16u, FLAG_OFFSETS_32 = 32u, FLAG_PAIR_COLUMNS = 64u, FLAG_PAIR_TILES = 128u, FLAG_QUAD_FILL = 256u };
+// FLAG_GROUP_IO: a thread's K pixels move as wide accesses, at whatever byte alignment; FLAG_VECTOR_IO: at their natural
+// alignment as well
+enum : unsigned { FLAG_VECTOR_IO = 1u, FLAG_GROUP_IO = 512u, FLAG_STREAM_STORES = 2u, FLAG_SOURCE_TILE = 4u, FLAG_WHOLE_BOX = 8u, FLAG_PACKED_TILE = 16u, FLAG_OFFSETS_32 = 32u, FLAG_PAIR_COLUMNS = 64u, FLAG_PAIR_TILES = 128u, FLAG_QUAD_FILL = 256u };
 
 template <typename Prog, size_t N, typename Out, typename Defaults = NoDefaultPlanes>
 struct PointwiseJob {
@@ -578,14 +727,16 @@ struct PointwiseJob {
     using Access = SourceAccess<View>;
     using Src = typename View::Source;
     using OutPixel = typename Out::Pixel;
-    static constexpr int K = Access::template pixels<OutPixel, Out::IS_SPLIT>();
+    static constexpr int K = Access::template pixels<OutPixel, Out::IS_SPLIT>(); // pixels per thread and row
+    static constexpr int ROWS = Access::ROWS > Out::ROWS ? Access::ROWS : Out::ROWS; // rows per thread
+    using Group = typename Access::template Group<K>;
     static constexpr int IN_BYTES = K * static_cast<int>(sizeof(Src));
     static constexpr int OUT_BYTES = Out::IS_SPLIT ? K * static_cast<int>(sizeof(VBase<OutPixel>)) : K * static_cast<int>(sizeof(OutPixel));
     // A thread's K pixels span more than one 16-byte transaction when pixels are 12 bytes wide (48 bytes per thread).
-    // Lanes reading 48-byte runs touch every cache line three times; instead the block moves its contiguous span of up
-    // to 256*K pixels with fully coalesced 16-byte accesses and redistributes pixels to threads through LDS.
-    static constexpr bool STAGE_IN = Access::FLATTENS && IN_BYTES > 16 && IN_BYTES % 16 == 0;
-    static constexpr bool STAGE_OUT = !Out::IS_SPLIT && OUT_BYTES > 16 && OUT_BYTES % 16 == 0;
+    // Lanes reading 48-byte runs touch every cache line three times; instead a wave moves its contiguous span of up
+    // to 64*K pixels with fully coalesced 16-byte accesses and redistributes pixels to threads through LDS.
+    static constexpr bool STAGE_IN = Access::FLATTENS && ROWS == 1 && IN_BYTES > 16 && IN_BYTES % 16 == 0 && sizeof(Src) % 4 == 0;
+    static constexpr bool STAGE_OUT = !Out::IS_SPLIT && Out::ROW_MAJOR && OUT_BYTES > 16 && OUT_BYTES % 16 == 0 && sizeof(OutPixel) % 4 == 0;
     static constexpr int STAGE_BYTES = (STAGE_IN && STAGE_OUT) ? (IN_BYTES > OUT_BYTES ? IN_BYTES : OUT_BYTES)
                                        : STAGE_IN              ? IN_BYTES
                                        : STAGE_OUT             ? OUT_BYTES
@@ -600,78 +751,152 @@ struct PointwiseJob {
     Out out;
     unsigned tx_shift; // log2 of the thread columns of a block; the other threads cover further rows
     unsigned grid_x, grid_y;
-    unsigned pair_limit; // blocks that are re-dealt so that row pairs share an XCD (0: none)
     Defaults defaults;
     size_t lds_bytes() const { return LDS_BYTES; }
 
-    // A block that lies on one row and owns `span` pixels of it from pixel bx0 on (a whole number of thread groups, so
-    // the span is whole 16-byte pieces on both sides).  FULL: span is the block's whole 256*K pixels, nothing is guarded.
+    // The thread columns of a block for an image of `groups` thread groups by `rows` thread rows: of 64, 128 and 256 the count that
+    // leaves the fewest threads without pixels (3840 pixels of four per thread are 960 groups: 256 columns idle one thread in
+    // sixteen, 64 none), the larger one where several do.  Fewer than 64 (down to 16) only where a row has no more groups: a wave
+    // on several rows writes short pieces of each (3494 x 2014 pixels into an NV21 image: 11.5 us in columns of 16, 8.3 us of 64).
+    void plan(const unsigned groups, const unsigned rows) {
+        unsigned narrowest = 4u;
+        while (narrowest < 6u && (1u << narrowest) < groups) ++narrowest;
+        size_t least = ~static_cast<size_t>(0);
+        for (unsigned shift = narrowest; shift <= 8u; ++shift) {
+            const unsigned cols = 1u << shift, lines = BLOCK_THREADS >> shift;
+            const unsigned gx = (groups + cols - 1u) / cols, gy = (rows + lines - 1u) / lines;
+            const size_t blocks = static_cast<size_t>(gx) * gy;
+            if (blocks <= least) {
+                least = blocks;
+                tx_shift = shift;
+                grid_x = gx;
+                grid_y = gy;
+            }
+        }
+    }
+
+    // The source pixels of a thread, row by row, handed to emit(row as a constant, group).  `whole`: the K pixels exist.  Only
+    // the loads depend on it, so that an emit of the whole wave stays one even where some lanes' groups are cut.
+    template <typename Emit>
+    __device__ __attribute__((always_inline)) static inline void each_row(const View& v, const bool whole, const bool whole_box, int x0, int y, const Emit& emit) {
+        const auto load = [&](const int row, Group& in) {
+            if (whole) Access::template load_group<K>(v, x0, row, in);
+            else Access::template load_each<K>(v, whole_box, x0, row, in);
+        };
+        const bool two = ROWS == 2 && y + 1 < v.h;
+        if constexpr (ROWS == 1) {
+            Group in;
+            load(y, in);
+            emit(std::integral_constant<int, 0>{}, in);
+        } else {
+            if constexpr (Access::ROWS == 2) {
+                if ((v.oy & 1) != 0) { // rows y and y + 1 of the window are not a row pair of the image
+                    Group in;
+                    load(y, in);
+                    emit(std::integral_constant<int, 0>{}, in);
+                    if (two) {
+                        load(y + 1, in);
+                        emit(std::integral_constant<int, 1>{}, in);
+                    }
+                    return;
+                }
+            }
+            Group upper, lower;
+            const int below = two ? y + 1 : y;
+            if constexpr (Access::ROWS == 2) {
+                if (whole) Access::template load_group_pair<K>(v, x0, y, below, upper, lower);
+                else Access::template load_each_pair<K>(v, x0, y, below, upper, lower);
+            } else {
+                load(y, upper);
+                load(below, lower);
+            }
+            emit(std::integral_constant<int, 0>{}, upper);
+            if (two) emit(std::integral_constant<int, 1>{}, lower);
+        }
+    }
+
+    // A wave that lies on one row (or row pair) and owns `span` pixels of it from pixel wx0 on.  FULL: span is the wave's
+    // whole 64*K pixels, nothing is guarded.  The wave moves its span through its own part of the buffer and never waits for
+    // the other waves of the block.
     template <bool FULL>
-    __device__ __attribute__((always_inline)) static inline void row_block(const Out& job_out, const Plane& pl, const View& v, const unsigned pl_flags, int bx0, int span,
+    __device__ __attribute__((always_inline)) static inline void wave_span(const Out& job_out, const Plane& pl, const View& v, const unsigned pl_flags, int wx0, int span,
                                                                           int x0, int y, unsigned bz, int tid, unsigned char* lds) {
-        // A wave's 64 threads own 64*K consecutive pixels, so a wave moves its own span through its own part of the
-        // buffer and never waits for the other waves of the block.
         const int wave = tid >> 6, lane = tid & 63;
         dev::u32x4* const stage = reinterpret_cast<dev::u32x4*>(lds) + wave * (64 * STAGE_BYTES / 16);
         const bool active = FULL || x0 < v.w;
-        Src in[K];
+        const auto emit = [&](const auto row, const Group& in) {
+            const int yr = y + decltype(row)::value;
+            OutPixel o[K];
+            if (active) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
+            }
+            if constexpr (STAGE_OUT) {
+                constexpr int MINE = OUT_BYTES / 16;
+                if constexpr (STAGE_IN || ROWS > 1) dev::wave_sync(); // every lane has taken what it needs out of the buffer
+                if (active) {
+                    unsigned int w[OUT_BYTES / 4];
+                    dev::pack_pixels<K>(o, w);
+#pragma unroll
+                    for (int j = 0; j < MINE; ++j) {
+                        dev::u32x4 piece;
+                        piece.x = w[4 * j]; piece.y = w[4 * j + 1]; piece.z = w[4 * j + 2]; piece.w = w[4 * j + 3];
+                        stage[lane * MINE + j] = piece;
+                    }
+                }
+                dev::wave_sync();
+                char* const g = reinterpret_cast<char*>(job_out.data) + static_cast<size_t>(bz) * job_out.z_stride +
+                                static_cast<size_t>(yr) * job_out.pitch + static_cast<size_t>(wx0) * sizeof(OutPixel);
+                const int dwords = span * static_cast<int>(sizeof(OutPixel) / 4), pieces = dwords >> 2;
+                const unsigned int* const rest = reinterpret_cast<const unsigned int*>(stage);
+                if ((pl_flags & FLAG_STREAM_STORES) != 0u) {
+                    // the wave's span starts at the same address for all its lanes
+                    const __amdgpu_buffer_rsrc_t span_buffer = dev::wave_buffer(dev::wave_uniform(g));
+#pragma unroll
+                    for (int j = 0; j < MINE; ++j) {
+                        if (FULL || j * 64 + lane < pieces) dev::stream_store_at<4>(span_buffer, static_cast<unsigned>(j * 64 + lane) * 16u, 0u, stage[j * 64 + lane]);
+                    }
+                    if (!FULL && lane < dwords - 4 * pieces) dev::stream_store_at<1>(span_buffer, static_cast<unsigned>(4 * pieces + lane) * 4u, 0u, rest[4 * pieces + lane]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < MINE; ++j) {
+                        if (FULL || j * 64 + lane < pieces) dev::store_piece(g + (j * 64 + lane) * 16, stage[j * 64 + lane]);
+                    }
+                    if (!FULL && lane < dwords - 4 * pieces) dev::store_words<4>(g + (4 * pieces + lane) * 4, rest + 4 * pieces + lane);
+                }
+            } else if (active) {
+                if (FULL || x0 + K <= v.w) {
+                    dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        if (x0 + k < v.w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
+                    }
+                }
+            }
+        };
         if constexpr (STAGE_IN) {
             constexpr int MINE = IN_BYTES / 16;
-            const dev::u32x4* const g =
-                reinterpret_cast<const dev::u32x4*>(Access::row(v, y) + static_cast<size_t>(bx0) * sizeof(Src)) + wave * (64 * MINE);
-            const int pieces = span * static_cast<int>(sizeof(Src)) / 16 - wave * (64 * MINE); // of this wave's span
+            const char* const g = Access::row(v, y) + static_cast<size_t>(wx0) * sizeof(Src);
+            const int dwords = span * static_cast<int>(sizeof(Src) / 4), pieces = dwords >> 2;
 #pragma unroll
             for (int j = 0; j < MINE; ++j) {
-                if (FULL || j * 64 + lane < pieces) stage[j * 64 + lane] = g[j * 64 + lane];
+                if (FULL || j * 64 + lane < pieces) stage[j * 64 + lane] = dev::load_piece(g + (j * 64 + lane) * 16);
             }
+            if (!FULL && lane < dwords - 4 * pieces) dev::load_words<4>(g + (4 * pieces + lane) * 4, reinterpret_cast<unsigned int*>(stage) + 4 * pieces + lane);
             dev::wave_sync();
+            Group in;
             if (active) {
-                dev::u32x4 mine[MINE];
 #pragma unroll
-                for (int j = 0; j < MINE; ++j) mine[j] = stage[lane * MINE + j];
-                __builtin_memcpy(in, mine, IN_BYTES);
+                for (int j = 0; j < MINE; ++j) {
+                    const dev::u32x4 piece = stage[lane * MINE + j];
+                    in.w[4 * j] = piece.x; in.w[4 * j + 1] = piece.y; in.w[4 * j + 2] = piece.z; in.w[4 * j + 3] = piece.w;
+                }
             }
+            emit(std::integral_constant<int, 0>{}, in);
         } else {
-            if (active) Access::template load_group<K>(v, x0, y, in);
-        }
-        OutPixel o[K];
-        if (active) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in[k]);
-        }
-        if constexpr (STAGE_OUT) {
-            constexpr int MINE = OUT_BYTES / 16;
-            if constexpr (STAGE_IN) dev::wave_sync(); // every lane has taken its input out of the buffer
-            if (active) {
-                unsigned int w[OUT_BYTES / 4];
-                dev::pack_pixels<K>(o, w);
-#pragma unroll
-                for (int j = 0; j < MINE; ++j) {
-                    dev::u32x4 piece;
-                    piece.x = w[4 * j]; piece.y = w[4 * j + 1]; piece.z = w[4 * j + 2]; piece.w = w[4 * j + 3];
-                    stage[lane * MINE + j] = piece;
-                }
-            }
-            dev::wave_sync();
-            dev::u32x4* const g = reinterpret_cast<dev::u32x4*>(
-                reinterpret_cast<char*>(job_out.data) + static_cast<size_t>(bz) * job_out.z_stride +
-                static_cast<size_t>(y) * job_out.pitch + static_cast<size_t>(bx0) * sizeof(OutPixel)) + wave * (64 * MINE);
-            const int pieces = span * static_cast<int>(sizeof(OutPixel)) / 16 - wave * (64 * MINE);
-            if ((pl_flags & FLAG_STREAM_STORES) != 0u) {
-                // the wave's span starts at the same address for all its lanes
-                const __amdgpu_buffer_rsrc_t span_buffer = dev::wave_buffer(dev::wave_uniform(reinterpret_cast<char*>(g)));
-#pragma unroll
-                for (int j = 0; j < MINE; ++j) {
-                    if (FULL || j * 64 + lane < pieces) dev::stream_store_at<4>(span_buffer, static_cast<unsigned>(j * 64 + lane) * 16u, 0u, stage[j * 64 + lane]);
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < MINE; ++j) {
-                    if (FULL || j * 64 + lane < pieces) g[j * 64 + lane] = stage[j * 64 + lane];
-                }
-            }
-        } else if (active) {
-            dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, y, static_cast<int>(bz), o);
+            const int xl = active ? x0 : wx0; // (lanes past the row's end repeat the wave's first group and store nothing)
+            each_row(v, FULL || xl + K <= v.w, false, xl, y, emit);
         }
     }
 
@@ -679,8 +904,11 @@ struct PointwiseJob {
         if constexpr (Defaults::ENABLED) {
             if (bz >= job.defaults.used) {
                 const int cols = 1 << job.tx_shift, t = dev::thread_in_block();
-                dev::fill_default(job.out, job.defaults, (static_cast<int>(bx) * cols + (t & (cols - 1))) * K, K,
-                                  static_cast<int>(by) * (BLOCK_THREADS >> job.tx_shift) + (t >> job.tx_shift), static_cast<int>(bz));
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    dev::fill_default(job.out, job.defaults, (static_cast<int>(bx) * cols + (t & (cols - 1))) * K, K,
+                                      (static_cast<int>(by) * (BLOCK_THREADS >> job.tx_shift) + (t >> job.tx_shift)) * ROWS + r, static_cast<int>(bz));
+                }
                 return;
             }
         }
@@ -689,25 +917,12 @@ struct PointwiseJob {
         // the other); the tail stays where it is and is read while the pixels are on their way.
         const Plane& pl = job.plane[N == 1 ? 0u : bz];
         const View v = pl.prog.view;
-        const unsigned pl_flags = pl.flags, job_grid_x = job.grid_x, job_pair_limit = job.pair_limit, job_tx_shift = job.tx_shift;
+        const unsigned pl_flags = pl.flags, job_tx_shift = job.tx_shift;
         const Out job_out = job.out;
         const int tid = dev::thread_in_block();
-        // pair_limit != 0 (one row per block row, the source shares a chroma row between rows 2k and 2k + 1): workgroups go
-        // to the eight XCDs round-robin in launch order, so blocks b and b + 8 run on the same XCD one after the other.
-        // Giving them the same columns of rows 2k and 2k + 1 lets the second find the chroma row in that XCD's L2 instead
-        // of fetching it from memory again through another one.  The first pair_limit blocks (a multiple of 16 and of two
-        // block rows) are dealt out that way among themselves; the few after them keep their places.
-        const unsigned launch_index = bx + job_grid_x * by;
-        if (launch_index < job_pair_limit) {
-            const unsigned xcd = launch_index & 7u, turn = launch_index >> 3;
-            const unsigned pair = 8u * (turn >> 1) + xcd; // (columns, row pair) in the order the XCDs take them up
-            const unsigned k = pair / job_grid_x;
-            bx = pair - k * job_grid_x;
-            by = 2u * k + (turn & 1u);
-        }
         const int cols = 1 << job_tx_shift;
         const int x0 = (static_cast<int>(bx) * cols + (tid & (cols - 1))) * K;
-        const int y = static_cast<int>(by) * (BLOCK_THREADS >> job_tx_shift) + (tid >> job_tx_shift);
+        const int y = (static_cast<int>(by) * (BLOCK_THREADS >> job_tx_shift) + (tid >> job_tx_shift)) * ROWS;
 
         // FLAG_WHOLE_BOX (a batch of windows of different sizes): every plane produces the extent of the largest, as the
         // reference's thread grid does (batch_operations.h:153-160), so v.w x v.h is that box and elements beside the
@@ -715,41 +930,45 @@ struct PointwiseJob {
         // is zero.
         bool whole_box = false;
         if constexpr (std::is_same_v<View, PlainView<Src>>) whole_box = (pl_flags & FLAG_WHOLE_BOX) != 0u;
-        if constexpr (STAGE_IN || STAGE_OUT) {
-            // block-uniform decisions
-            const int bx0 = static_cast<int>(bx) * BLOCK_THREADS * K; // first pixel of the block
-            const int span = v.w - bx0 < BLOCK_THREADS * K ? v.w - bx0 : BLOCK_THREADS * K;
-            if ((pl_flags & FLAG_VECTOR_IO) != 0u && !whole_box && job_tx_shift == 8u && y < v.h && span > 0 && span % K == 0) {
-                if (span == BLOCK_THREADS * K) row_block<true>(job_out, pl, v, pl_flags, bx0, span, x0, y, bz, tid, lds);
-                else row_block<false>(job_out, pl, v, pl_flags, bx0, span, x0, y, bz, tid, lds);
-                return;
-            }
+        // (wave-uniform decisions: a wave of 64 thread columns lies on one row)
+        if ((pl_flags & FLAG_GROUP_IO) != 0u && !whole_box && job_tx_shift >= 6u) {
+            const int wx0 = __builtin_amdgcn_readfirstlane(x0), wy = __builtin_amdgcn_readfirstlane(y);
+            const int span = v.w - wx0 < 64 * K ? v.w - wx0 : 64 * K;
+            if (wy >= v.h || span <= 0) return;
+            if (span == 64 * K) wave_span<true>(job_out, pl, v, pl_flags, wx0, span, x0, wy, bz, tid, lds);
+            else wave_span<false>(job_out, pl, v, pl_flags, wx0, span, x0, wy, bz, tid, lds);
+            return;
         }
 
         if (y >= v.h || x0 >= v.w) return;
-        bool run_in_parent = true; // the thread's K pixels lie in the parent image
-        if constexpr (std::is_same_v<View, PlainView<Src>>) {
-            if (whole_box) run_in_parent = v.oy + y < v.img_h && v.ox + x0 + K <= v.img_w;
-        }
-        if ((pl_flags & FLAG_VECTOR_IO) != 0u && x0 + K <= v.w && run_in_parent) {
-            Src in[K];
-            Access::template load_group<K>(v, x0, y, in);
-            OutPixel o[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in[k]);
-            dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, y, static_cast<int>(bz), o);
-        } else {
-            const int xe = x0 + K < v.w ? x0 + K : v.w;
-            for (int x = x0; x < xe; ++x) {
-                Src pixel{};
-                bool in_parent = true;
-                if constexpr (std::is_same_v<View, PlainView<Src>>) {
-                    if (whole_box) in_parent = v.oy + y < v.img_h && v.ox + x < v.img_w;
+        if constexpr (!std::is_same_v<View, PlainView<Src>>) {
+            if ((pl_flags & FLAG_GROUP_IO) == 0u) { // a window that begins inside a chroma pair: pixel by pixel
+                for (int r = 0; r < ROWS && y + r < v.h; ++r) {
+                    for (int x = x0; x < x0 + K && x < v.w; ++x) {
+                        dev::store_one(job_out, x, y + r, static_cast<int>(bz), dev::apply_tail(pl.prog.tail, Access::load_one(v, x, y + r)));
+                    }
                 }
-                if (in_parent) pixel = Access::load_one(v, x, y);
-                dev::store_one(job_out, x, y, static_cast<int>(bz), dev::apply_tail(pl.prog.tail, pixel));
+                return;
             }
         }
+        bool whole = x0 + K <= v.w; // the thread's K pixels exist
+        if constexpr (std::is_same_v<View, PlainView<Src>>) {
+            if (whole_box) whole = whole && v.oy + y + ROWS <= v.img_h && v.ox + x0 + K <= v.img_w;
+        }
+        each_row(v, whole, whole_box, x0, y, [&](const auto row, const Group& in) {
+            const int yr = y + decltype(row)::value;
+            OutPixel o[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
+            if (x0 + K <= v.w) {
+                dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
+            } else {
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    if (x0 + k < v.w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
+                }
+            }
+        });
     }
 };
 

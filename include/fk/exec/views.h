@@ -309,6 +309,8 @@ template <typename O>
 struct PackedOut {
     using Pixel = O;
     static constexpr bool IS_SPLIT = false;
+    static constexpr bool ROW_MAJOR = true; // the pixels of a row are one run of bytes
+    static constexpr int ROWS = 1;          // rows that are best written together
     O* data;
     uint pitch;
     size_t z_stride; // bytes between planes
@@ -318,15 +320,44 @@ template <typename O>
 struct SplitOut {
     using Pixel = O;
     static constexpr bool IS_SPLIT = true;
+    static constexpr bool ROW_MAJOR = false;
+    static constexpr int ROWS = 1;
     VBase<O>* data;
     uint pitch;
     size_t z_stride;
     size_t chan_stride; // bytes between channel planes
 };
 
+// {Y, U, V} pixels into a raw YUV image; in a 4:2:0 format a row pair writes one chroma row.
+template <PixelFormat PF>
+struct YuvOut {
+    using Base = ColorDepthPixelBaseType<PixelFormatTraits<PF>::depth>;
+    using Pixel = typename WriteYUV<PF>::InputType;
+    static constexpr bool IS_SPLIT = false;
+    static constexpr bool ROW_MAJOR = false;
+    static constexpr int rows_together() {
+        if constexpr (fk::detail::YuvLayout<PF>::semi_planar) return fk::detail::YuvLayout<PF>::row_shift == 1 ? 2 : 1;
+        else return 1;
+    }
+    static constexpr int ROWS = rows_together();
+    Base* data;
+    uint pitch;
+    uint img_w, img_h; // chroma rows follow row img_h - 1
+    size_t z_stride;   // 0: one image
+};
+
 template <typename IOp>
 struct OutOf {
     static constexpr bool supported = false;
+};
+template <PixelFormat PF>
+struct OutOf<Write<WriteYUV<PF>>> {
+    static constexpr bool supported = true;
+    using type = YuvOut<PF>;
+    static type make(const Write<WriteYUV<PF>>& iOp) {
+        const RawImage<PF>& raw = iOp.params;
+        return type{ raw.data.data, raw.data.dims.pitch, static_cast<uint>(raw.width), static_cast<uint>(raw.height), 0 };
+    }
 };
 template <typename O>
 struct OutOf<Write<PerThreadWrite<ND::_2D, O>>> {

@@ -1,0 +1,79 @@
+// YUV images as sources and receivers of element-wise chains at every parity of origin and size, as user code: each chain runs
+// through the GPU executor and, on the host, through TransformDPP<ParArch::CPU>; the results are compared byte for byte.
+#include <fused_kernel/fused_kernel.h>
+
+#include <cstdio>
+#include <cstring>
+
+using namespace fk;
+
+static int failures = 0;
+
+template <typename T>
+static bool same_rows(const Ptr2D<T>& a, const Ptr2D<T>& b) {
+    for (uint y = 0; y < a.dims().height; ++y)
+        for (uint x = 0; x < a.dims().width; ++x) {
+            const T p = a.at(x, y), q = b.at(x, y);
+            if (std::memcmp(&p, &q, sizeof(T)) != 0) return false;
+        }
+    return true;
+}
+
+template <PixelFormat PF>
+static void check(const char* name, Stream& stream) {
+    using Base = typename Image<PF>::BaseType;
+    using Pixel = typename ReadYUV<PF>::OutputType;
+    Stream_<ParArch::CPU> host_stream;
+    constexpr ResolutionFactors rf = PixelFormatTraits<PF>::rf;
+    const uint w = 544, h = 22;
+    Ptr2D<Base> data(static_cast<uint>(w * rf.width_f), static_cast<uint>(h * rf.height_f));
+    for (uint y = 0; y < data.dims().height; ++y)
+        for (uint x = 0; x < data.dims().width; ++x) data.at(x, y) = static_cast<Base>((x * 7919u + y * 104729u) ^ (x * y));
+    data.upload(stream);
+    const Image<PF> image(data, w, h);
+    RawImage<PF> on_host = image.ptr();
+    on_host.data = data.ptrPinned();
+    for (int oy = 0; oy < 2; ++oy)
+        for (int ox = 0; ox < 2; ++ox)
+            for (int dh = 0; dh < 2; ++dh)
+                for (int cw : { 1, 3, 64, 257, 530 }) {
+                    const Rect window(static_cast<uint>(ox), static_cast<uint>(oy), cw, 18 + dh);
+                    Ptr2D<Pixel> gpu(static_cast<uint>(cw), static_cast<uint>(18 + dh)), cpu(static_cast<uint>(cw), static_cast<uint>(18 + dh), 0, MemType::Host);
+                    executeOperations<TransformDPP<>>(stream, ReadYUV<PF>::build(image).then(Crop<>::build(window)), PerThreadWrite<ND::_2D, Pixel>::build(gpu));
+                    gpu.download(stream);
+                    stream.sync();
+                    executeOperations<TransformDPP<ParArch::CPU>>(host_stream, ReadYUV<PF>::build(on_host).then(Crop<>::build(window)), PerThreadWrite<ND::_2D, Pixel>::build(cpu));
+                    if (!same_rows(gpu, cpu)) {
+                        std::printf("FAILED %s: window %d,%d %dx%d\n", name, ox, oy, cw, 18 + dh);
+                        ++failures;
+                    }
+                    // and back: the pixels into an image of that size, odd sizes included
+                    const uint rows = static_cast<uint>((18 + dh + 1) * rf.height_f), cols = static_cast<uint>((cw + 1) * rf.width_f);
+                    Ptr2D<Base> raw_gpu(cols, rows), raw_cpu(cols, rows, 0, MemType::Host);
+                    for (uint y = 0; y < rows; ++y)
+                        for (uint x = 0; x < cols; ++x) raw_gpu.at(x, y) = raw_cpu.at(x, y) = static_cast<Base>(77);
+                    raw_gpu.upload(stream);
+                    const RawImage<PF> to_gpu{ raw_gpu.ptr(), static_cast<uint>(cw), static_cast<uint>(18 + dh) };
+                    const RawImage<PF> to_cpu{ raw_cpu.ptr(), static_cast<uint>(cw), static_cast<uint>(18 + dh) };
+                    executeOperations<TransformDPP<>>(stream, PerThreadRead<ND::_2D, Pixel>::build(gpu.ptr()), WriteYUV<PF>::build(to_gpu));
+                    raw_gpu.download(stream);
+                    stream.sync();
+                    executeOperations<TransformDPP<ParArch::CPU>>(host_stream, PerThreadRead<ND::_2D, Pixel>::build(cpu.ptr()), WriteYUV<PF>::build(to_cpu));
+                    if (!same_rows(raw_gpu, raw_cpu)) {
+                        std::printf("FAILED %s: receiver %dx%d\n", name, cw, 18 + dh);
+                        ++failures;
+                    }
+                }
+}
+
+int main() {
+    Stream stream;
+    check<PixelFormat::NV12>("NV12", stream);
+    check<PixelFormat::NV21>("NV21", stream);
+    check<PixelFormat::P010>("P010", stream);
+    check<PixelFormat::P210>("P210", stream);
+    check<PixelFormat::Y210>("Y210", stream);
+    check<PixelFormat::UYVY>("UYVY", stream);
+    if (failures == 0) std::printf("yuv_windows ok\n");
+    return failures == 0 ? 0 : 1;
+}

@@ -1,0 +1,86 @@
+"""Element-wise chains whose rows start at any byte: a thread moves a group of pixels with wide accesses whatever the alignment,
+a wave of 64 groups lies on one row (on a row pair of a 4:2:0 image), and the last group of a row may be cut.  Widths around a
+wave's span (256 pixels of four per thread, 128 of two), groups cut at every even place, images that start between dwords, and
+bytes beside every row that must stay as they were; against the CPU oracle, bit for bit."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import same_bits
+from oracle import binding as B
+
+pytestmark = pytest.mark.gpu
+FILL = 85
+
+
+def window(a, left, right):
+    """`a` (h, w[, c]) in device memory with `left` and `right` extra columns beside every row, filled with a pattern."""
+    a = np.ascontiguousarray(a)
+    a = a.view(np.int16) if a.dtype == np.uint16 else a
+    big = np.full((a.shape[0], left + a.shape[1] + right) + a.shape[2:], FILL, a.dtype)
+    big[:, left:left + a.shape[1]] = a
+    t = torch.from_numpy(big).cuda()
+    return t, t[:, left:left + a.shape[1]]
+
+
+def host(t, dt):
+    a = np.ascontiguousarray(t.cpu().numpy())
+    return a.view(np.uint16) if dt == np.uint16 else a
+
+
+def untouched_beside(big, left, width):
+    return bool((big[:, :left] == FILL).all()) and bool((big[:, left + width:] == FILL).all())
+
+
+@pytest.mark.parametrize("name", list(B.YUV_FORMATS))
+@pytest.mark.parametrize("w,h,left,right", [(126, 6, 0, 0), (130, 2, 1, 0), (254, 4, 3, 2), (256, 2, 0, 1), (258, 6, 2, 1), (262, 4, 1, 2), (1030, 2, 0, 3), (34, 18, 1, 1), (2, 2, 1, 0)])
+def test_yuv_rows_at_any_byte(fk, oracle, name, w, h, left, right):
+    fmt = B.YUV_FORMATS[name]
+    rows, cols, dt = oracle.yuv_data_shape(fmt, w, h)
+    dt = np.dtype(dt).type
+    raw = oracle.bytes(700 + w, (rows, cols * np.dtype(dt).itemsize)).view(dt)
+    _, d_raw = window(raw, left, right)
+    # unpack and convert
+    big, out = window(np.zeros((h, w, 3), dt), left, right)
+    fk.read_yuv(fmt, d_raw, out)
+    assert same_bits(host(out, dt), oracle.read_yuv(fmt, raw, w, h)) and untouched_beside(big, left, w)
+    rng, prim = B.YUV_MATRICES[w % 4]
+    for alpha, float_out in ((0, 0), (1, 0), (0, 1), (1, 1)):
+        odt = np.float32 if float_out else dt
+        big, out = window(np.zeros((h, w, 4 if alpha else 3), odt), left, right)
+        fk.yuv_to_rgb(fmt, rng, prim, d_raw, out)
+        assert same_bits(host(out, odt), oracle.yuv_to_rgb(fmt, rng, prim, alpha, float_out, raw, w, h)) and untouched_beside(big, left, w), (alpha, float_out)
+    # pack
+    pixels = oracle.bytes(710 + w, (h, w * 3 * np.dtype(dt).itemsize)).view(dt).reshape(h, w, 3)
+    big, written = window(np.zeros_like(raw), left, right)
+    fk.write_yuv(fmt, window(pixels, left, right)[1], written)
+    assert same_bits(host(written, dt), oracle.write_yuv(fmt, pixels)) and untouched_beside(big, left, cols)
+
+
+@pytest.mark.parametrize("w,h,left,right", [(255, 3, 1, 0), (257, 2, 0, 1), (259, 5, 2, 3), (1023, 2, 1, 1), (61, 9, 3, 0), (3, 3, 1, 2), (1, 1, 0, 0)])
+def test_plain_rows_at_any_pixel(fk, oracle, w, h, left, right):
+    """Chains over four-byte and twelve-byte pixels: the spans that leave through LDS end in whole dwords, not whole pieces."""
+    src4 = oracle.bytes(720 + w, (h, w, 4))
+    _, d4 = window(src4, left, right)
+    big, gray = window(np.zeros((h, w), np.uint8), left, right)
+    fk.rgba2gray_u8c4(d4, gray)
+    assert same_bits(gray.cpu().numpy(), oracle.rgba2gray_u8c4(src4)) and untouched_beside(big, left, w)
+    big, bgr = window(np.zeros((h, w, 3), np.float32), left, right)
+    fk.rgba2bgr_sub_u8c4_f32c3(d4, bgr, 0.5)
+    assert same_bits(bgr.cpu().numpy(), oracle.rgba2bgr_sub_u8c4_f32c3(src4, 0.5)) and untouched_beside(big, left, w)
+    src = oracle.unit_floats(730 + w, (h, w, 3))
+    big, out = window(np.zeros((h, w, 3), np.float32), left, right)
+    fk.muladd_chain_f32c3(window(src, left, right)[1], out, 4, 1.0001, 1e-4)
+    assert same_bits(out.cpu().numpy(), oracle.muladd_chain_f32c3(src, 4, 1.0001, 1e-4)) and untouched_beside(big, left, w)
+
+
+def test_windows_at_odd_rows_and_columns_as_user_code():
+    """Crops of YUV images at every parity of their origin and size, and YUV images of odd size as receivers, through the GPU
+    executor and the host executor of the operator API: the same bits."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "yuv_windows")
+    assert os.path.exists(exe), "tests/cpp/yuv_windows is not built"
+    proc = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert proc.returncode == 0 and "yuv_windows ok" in proc.stdout, proc.stdout
