@@ -525,9 +525,11 @@ private:
         using Plan = exec::JobOf<std::decay_t<decltype(seq.sender)>, std::decay_t<decltype(seq.receiver)>>;
         pack.job = Plan::make(seq.sender, seq.receiver);
         pack.blocks = pack.job.grid_x * pack.job.grid_y * Plan::planes(seq.sender);
+        pack.twin = 0u;
         total += pack.blocks;
         lds = lds > pack.job.lds_bytes() ? lds : pack.job.lds_bytes();
         fill(pack.rest, total, lds, rest...);
+        total -= pack.pair_up(); // (the jobs behind it are filled in)
     }
 };
 

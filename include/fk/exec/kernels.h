@@ -721,6 +721,10 @@ __device__ __attribute__((always_inline)) inline void fill_default(const Out& ou
 // alignment as well
 enum : unsigned { FLAG_VECTOR_IO = 1u, FLAG_GROUP_IO = 512u, FLAG_STREAM_STORES = 2u, FLAG_SOURCE_TILE = 4u, FLAG_WHOLE_BOX = 8u, FLAG_PACKED_TILE = 16u, FLAG_OFFSETS_32 = 32u, FLAG_PAIR_COLUMNS = 64u, FLAG_PAIR_TILES = 128u, FLAG_QUAD_FILL = 256u };
 
+constexpr int max_of(const int a) { return a; }
+template <typename... Rest>
+constexpr int max_of(const int a, const int b, const Rest... rest) { return max_of(a > b ? a : b, rest...); }
+
 template <typename Prog, size_t N, typename Out, typename Defaults = NoDefaultPlanes>
 struct PointwiseJob {
     using View = decltype(Prog::view);
@@ -730,6 +734,7 @@ struct PointwiseJob {
     static constexpr int K = Access::template pixels<OutPixel, Out::IS_SPLIT>(); // pixels per thread and row
     static constexpr int ROWS = Access::ROWS > Out::ROWS ? Access::ROWS : Out::ROWS; // rows per thread
     using Group = typename Access::template Group<K>;
+    static constexpr size_t PLANES = N;
     static constexpr int IN_BYTES = K * static_cast<int>(sizeof(Src));
     static constexpr int OUT_BYTES = Out::IS_SPLIT ? K * static_cast<int>(sizeof(VBase<OutPixel>)) : K * static_cast<int>(sizeof(OutPixel));
     // A thread's K pixels span more than one 16-byte transaction when pixels are 12 bytes wide (48 bytes per thread).
@@ -815,66 +820,81 @@ struct PointwiseJob {
         }
     }
 
-    // A wave that lies on one row (or row pair) and owns `span` pixels of it from pixel wx0 on.  FULL: span is the wave's
-    // whole 64*K pixels, nothing is guarded.  The wave moves its span through its own part of the buffer and never waits for
-    // the other waves of the block.
+    // One row of a wave's span through this job's tail into this job's output; `stage` is the wave's part of the buffer.
     template <bool FULL>
-    __device__ __attribute__((always_inline)) static inline void wave_span(const Out& job_out, const Plane& pl, const View& v, const unsigned pl_flags, int wx0, int span,
-                                                                          int x0, int y, unsigned bz, int tid, unsigned char* lds) {
-        const int wave = tid >> 6, lane = tid & 63;
-        dev::u32x4* const stage = reinterpret_cast<dev::u32x4*>(lds) + wave * (64 * STAGE_BYTES / 16);
-        const bool active = FULL || x0 < v.w;
-        const auto emit = [&](const auto row, const Group& in) {
-            const int yr = y + decltype(row)::value;
-            OutPixel o[K];
+    __device__ __attribute__((always_inline)) static inline void emit_span(const Out& job_out, const Plane& pl, const unsigned pl_flags, const Group& in, const bool active, int w,
+                                                                          int wx0, int span, int x0, int yr, unsigned bz, int lane, dev::u32x4* stage) {
+        OutPixel o[K];
+        if (active) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
+        }
+        if constexpr (STAGE_OUT) {
+            constexpr int MINE = OUT_BYTES / 16;
+            dev::wave_sync(); // every lane has taken what it needs out of the buffer
             if (active) {
+                unsigned int words[OUT_BYTES / 4];
+                dev::pack_pixels<K>(o, words);
 #pragma unroll
-                for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
-            }
-            if constexpr (STAGE_OUT) {
-                constexpr int MINE = OUT_BYTES / 16;
-                if constexpr (STAGE_IN || ROWS > 1) dev::wave_sync(); // every lane has taken what it needs out of the buffer
-                if (active) {
-                    unsigned int w[OUT_BYTES / 4];
-                    dev::pack_pixels<K>(o, w);
-#pragma unroll
-                    for (int j = 0; j < MINE; ++j) {
-                        dev::u32x4 piece;
-                        piece.x = w[4 * j]; piece.y = w[4 * j + 1]; piece.z = w[4 * j + 2]; piece.w = w[4 * j + 3];
-                        stage[lane * MINE + j] = piece;
-                    }
-                }
-                dev::wave_sync();
-                char* const g = reinterpret_cast<char*>(job_out.data) + static_cast<size_t>(bz) * job_out.z_stride +
-                                static_cast<size_t>(yr) * job_out.pitch + static_cast<size_t>(wx0) * sizeof(OutPixel);
-                const int dwords = span * static_cast<int>(sizeof(OutPixel) / 4), pieces = dwords >> 2;
-                const unsigned int* const rest = reinterpret_cast<const unsigned int*>(stage);
-                if ((pl_flags & FLAG_STREAM_STORES) != 0u) {
-                    // the wave's span starts at the same address for all its lanes
-                    const __amdgpu_buffer_rsrc_t span_buffer = dev::wave_buffer(dev::wave_uniform(g));
-#pragma unroll
-                    for (int j = 0; j < MINE; ++j) {
-                        if (FULL || j * 64 + lane < pieces) dev::stream_store_at<4>(span_buffer, static_cast<unsigned>(j * 64 + lane) * 16u, 0u, stage[j * 64 + lane]);
-                    }
-                    if (!FULL && lane < dwords - 4 * pieces) dev::stream_store_at<1>(span_buffer, static_cast<unsigned>(4 * pieces + lane) * 4u, 0u, rest[4 * pieces + lane]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < MINE; ++j) {
-                        if (FULL || j * 64 + lane < pieces) dev::store_piece(g + (j * 64 + lane) * 16, stage[j * 64 + lane]);
-                    }
-                    if (!FULL && lane < dwords - 4 * pieces) dev::store_words<4>(g + (4 * pieces + lane) * 4, rest + 4 * pieces + lane);
-                }
-            } else if (active) {
-                if (FULL || x0 + K <= v.w) {
-                    dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        if (x0 + k < v.w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
-                    }
+                for (int j = 0; j < MINE; ++j) {
+                    dev::u32x4 piece;
+                    piece.x = words[4 * j]; piece.y = words[4 * j + 1]; piece.z = words[4 * j + 2]; piece.w = words[4 * j + 3];
+                    stage[lane * MINE + j] = piece;
                 }
             }
-        };
+            dev::wave_sync();
+            char* const g = reinterpret_cast<char*>(job_out.data) + static_cast<size_t>(bz) * job_out.z_stride + static_cast<size_t>(yr) * job_out.pitch +
+                            static_cast<size_t>(wx0) * sizeof(OutPixel);
+            const int dwords = span * static_cast<int>(sizeof(OutPixel) / 4), pieces = dwords >> 2;
+            const unsigned int* const rest = reinterpret_cast<const unsigned int*>(stage);
+            if ((pl_flags & FLAG_STREAM_STORES) != 0u) {
+                // the wave's span starts at the same address for all its lanes
+                const __amdgpu_buffer_rsrc_t span_buffer = dev::wave_buffer(dev::wave_uniform(g));
+#pragma unroll
+                for (int j = 0; j < MINE; ++j) {
+                    if (FULL || j * 64 + lane < pieces) dev::stream_store_at<4>(span_buffer, static_cast<unsigned>(j * 64 + lane) * 16u, 0u, stage[j * 64 + lane]);
+                }
+                if (!FULL && lane < dwords - 4 * pieces) dev::stream_store_at<1>(span_buffer, static_cast<unsigned>(4 * pieces + lane) * 4u, 0u, rest[4 * pieces + lane]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < MINE; ++j) {
+                    if (FULL || j * 64 + lane < pieces) dev::store_piece(g + (j * 64 + lane) * 16, stage[j * 64 + lane]);
+                }
+                if (!FULL && lane < dwords - 4 * pieces) dev::store_words<4>(g + (4 * pieces + lane) * 4, rest + 4 * pieces + lane);
+            }
+        } else if (active) {
+            if (FULL || x0 + K <= w) {
+                dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
+            } else {
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    if (x0 + k < w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
+                }
+            }
+        }
+    }
+    // one row of a thread's group, the same without the buffer
+    __device__ __attribute__((always_inline)) static inline void emit_group(const Out& job_out, const Plane& pl, const unsigned pl_flags, const Group& in, int w, int x0, int yr,
+                                                                           unsigned bz) {
+        OutPixel o[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
+        if (x0 + K <= w) {
+            dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
+        } else {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                if (x0 + k < w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
+            }
+        }
+    }
+
+    // A wave that lies on one row (or row pair) and owns `span` pixels of it from pixel wx0 on, handed row by row to
+    // emit(row as a constant, group).  FULL: span is the wave's whole 64*K pixels, nothing is guarded.  The wave moves its span
+    // through its own part of the buffer and never waits for the other waves of the block.
+    template <bool FULL, typename Emit>
+    __device__ __attribute__((always_inline)) static inline void wave_span(const View& v, int wx0, int span, int x0, int y, int lane, dev::u32x4* stage, const Emit& emit) {
+        const bool active = FULL || x0 < v.w;
         if constexpr (STAGE_IN) {
             constexpr int MINE = IN_BYTES / 16;
             const char* const g = Access::row(v, y) + static_cast<size_t>(wx0) * sizeof(Src);
@@ -893,14 +913,29 @@ struct PointwiseJob {
                     in.w[4 * j] = piece.x; in.w[4 * j + 1] = piece.y; in.w[4 * j + 2] = piece.z; in.w[4 * j + 3] = piece.w;
                 }
             }
-            emit(std::integral_constant<int, 0>{}, in);
+            emit(std::integral_constant<int, 0>{}, in, active);
         } else {
             const int xl = active ? x0 : wx0; // (lanes past the row's end repeat the wave's first group and store nothing)
-            each_row(v, FULL || xl + K <= v.w, false, xl, y, emit);
+            each_row(v, FULL || xl + K <= v.w, false, xl, y, [&](const auto row, const Group& in) { emit(row, in, active); });
         }
     }
 
-    __device__ __attribute__((always_inline)) static inline void run(const PointwiseJob& job, unsigned bx, unsigned by, unsigned bz, unsigned char* lds) {
+    // Whether another job can take its pixels from this job's loads (JobPack): the same source window, dealt out to threads the
+    // same way.
+    template <typename Other, typename = void>
+    struct SharesSourceWith : std::false_type {};
+    template <typename Other>
+    struct SharesSourceWith<Other, std::void_t<typename Other::Group>>
+        : std::bool_constant<N == 1 && Other::PLANES == 1 && std::is_same_v<View, typename Other::View> && K == Other::K && ROWS == Other::ROWS && !Defaults::ENABLED> {};
+    template <typename Other>
+    bool shares_source_with(const Other& other) const {
+        return same_window(plane[0].prog.view, other.plane[0].prog.view) && tx_shift == other.tx_shift;
+    }
+
+    // `also`: further jobs (at most one plane each) that read the same window: a thread loads its pixels once and hands them to
+    // every job's tail and output.
+    template <typename... Also>
+    __device__ __attribute__((always_inline)) static inline void run(const PointwiseJob& job, unsigned bx, unsigned by, unsigned bz, unsigned char* lds, const Also&... also) {
         if constexpr (Defaults::ENABLED) {
             if (bz >= job.defaults.used) {
                 const int cols = 1 << job.tx_shift, t = dev::thread_in_block();
@@ -935,8 +970,19 @@ struct PointwiseJob {
             const int wx0 = __builtin_amdgcn_readfirstlane(x0), wy = __builtin_amdgcn_readfirstlane(y);
             const int span = v.w - wx0 < 64 * K ? v.w - wx0 : 64 * K;
             if (wy >= v.h || span <= 0) return;
-            if (span == 64 * K) wave_span<true>(job_out, pl, v, pl_flags, wx0, span, x0, wy, bz, tid, lds);
-            else wave_span<false>(job_out, pl, v, pl_flags, wx0, span, x0, wy, bz, tid, lds);
+            constexpr int WAVE_BYTES = 64 * max_of(STAGE_BYTES, Also::STAGE_BYTES...);
+            const int lane = tid & 63;
+            dev::u32x4* const stage = reinterpret_cast<dev::u32x4*>(lds) + (tid >> 6) * (WAVE_BYTES / 16);
+            const auto whole_wave = [&](const auto full) {
+                constexpr bool FULL = decltype(full)::value;
+                wave_span<FULL>(v, wx0, span, x0, wy, lane, stage, [&](const auto row, const Group& in, const bool active) {
+                    const int yr = wy + decltype(row)::value;
+                    emit_span<FULL>(job_out, pl, pl_flags, in, active, v.w, wx0, span, x0, yr, bz, lane, stage);
+                    (Also::template emit_span<FULL>(also.out, also.plane[0], also.plane[0].flags, in, active, v.w, wx0, span, x0, yr, 0u, lane, stage), ...);
+                });
+            };
+            if (span == 64 * K) whole_wave(std::true_type{});
+            else whole_wave(std::false_type{});
             return;
         }
 
@@ -945,7 +991,9 @@ struct PointwiseJob {
             if ((pl_flags & FLAG_GROUP_IO) == 0u) { // a window that begins inside a chroma pair: pixel by pixel
                 for (int r = 0; r < ROWS && y + r < v.h; ++r) {
                     for (int x = x0; x < x0 + K && x < v.w; ++x) {
-                        dev::store_one(job_out, x, y + r, static_cast<int>(bz), dev::apply_tail(pl.prog.tail, Access::load_one(v, x, y + r)));
+                        const Src pixel = Access::load_one(v, x, y + r);
+                        dev::store_one(job_out, x, y + r, static_cast<int>(bz), dev::apply_tail(pl.prog.tail, pixel));
+                        (dev::store_one(also.out, x, y + r, 0, dev::apply_tail(also.plane[0].prog.tail, pixel)), ...);
                     }
                 }
                 return;
@@ -956,18 +1004,8 @@ struct PointwiseJob {
             if (whole_box) whole = whole && v.oy + y + ROWS <= v.img_h && v.ox + x0 + K <= v.img_w;
         }
         each_row(v, whole, whole_box, x0, y, [&](const auto row, const Group& in) {
-            const int yr = y + decltype(row)::value;
-            OutPixel o[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) o[k] = dev::apply_tail(pl.prog.tail, in.pixel(k));
-            if (x0 + K <= v.w) {
-                dev::store_group_either<K>((pl_flags & FLAG_STREAM_STORES) != 0u, job_out, x0, yr, static_cast<int>(bz), o);
-            } else {
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    if (x0 + k < v.w) dev::store_one(job_out, x0 + k, yr, static_cast<int>(bz), o[k]);
-                }
-            }
+            emit_group(job_out, pl, pl_flags, in, v.w, x0, y + decltype(row)::value, bz);
+            (Also::emit_group(also.out, also.plane[0], also.plane[0].flags, in, v.w, x0, y + decltype(row)::value, 0u), ...);
         });
     }
 };
@@ -2051,6 +2089,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(BLOCK_THREADS, BLOCK_THREA
 
 // Several different jobs in one launch ("divergent horizontal fusion"): the 1-D grid is cut into one contiguous
 // range of blocks per job, sized to that job alone, so that a small job does not pay for a large one's grid.
+//
+// Two element-wise jobs over the same window of the same image (gray and BGR from one frame) are run by the blocks of the
+// first: a thread loads its pixels once and feeds both outputs (`twin`), and the second gets no blocks.  Four chains over
+// 8192 x 8192 uchar4, 1426 MB with the frame read by each of its two whole-frame jobs, 1158 MB with it read once: 210 -> 186 us.
+namespace dev {
+template <typename Job, typename Other, typename = void>
+struct SharesSource : std::false_type {};
+template <typename Job, typename Other>
+struct SharesSource<Job, Other, std::void_t<typename Job::template SharesSourceWith<Other>>> : Job::template SharesSourceWith<Other> {};
+} // namespace dev
 template <typename... Jobs>
 struct JobPack;
 template <>
@@ -2063,9 +2111,53 @@ struct JobPack<> {
 template <typename Job, typename... Rest>
 struct JobPack<Job, Rest...> {
     Job job;
-    unsigned blocks; // blocks of this job: grid_x * grid_y * planes
+    unsigned blocks; // blocks of this job: grid_x * grid_y * planes (0: the blocks of the job whose twin it is run it)
+    unsigned twin;   // P: this job's blocks run the P-th job after it as well (0: none)
     JobPack<Rest...> rest;
     static constexpr int COUNT = 1 + JobPack<Rest...>::COUNT;
+    // the pack that begins with the P-th job after this one
+    template <int P>
+    __host__ __device__ __attribute__((always_inline)) inline auto& after() {
+        if constexpr (P == 1) return rest;
+        else return rest.template after<P - 1>();
+    }
+    template <int P>
+    __host__ __device__ __attribute__((always_inline)) inline const auto& after() const {
+        if constexpr (P == 1) return rest;
+        else return rest.template after<P - 1>();
+    }
+    // Lets this job's blocks run another job as well where both read the same window; returns the blocks that this saves.
+    template <int P = 1>
+    unsigned pair_up() {
+        if constexpr (P < COUNT) {
+            auto& other = after<P>();
+            if constexpr (dev::SharesSource<Job, std::decay_t<decltype(other.job)>>::value) {
+                if (blocks != 0u && blocks == other.blocks && other.twin == 0u && job.shares_source_with(other.job)) {
+                    twin = static_cast<unsigned>(P);
+                    other.blocks = 0u;
+                    return blocks;
+                }
+            }
+            return pair_up<P + 1>();
+        } else {
+            return 0u;
+        }
+    }
+    template <int P>
+    __device__ __attribute__((always_inline)) static inline void run_with_twin(const JobPack& pack, unsigned bx, unsigned by, unsigned bz, unsigned char* lds) {
+        if constexpr (P < COUNT) {
+            using Other = std::decay_t<decltype(pack.template after<P>().job)>;
+            if constexpr (dev::SharesSource<Job, Other>::value) {
+                if (pack.twin == static_cast<unsigned>(P)) {
+                    Job::run(pack.job, bx, by, bz, lds, pack.template after<P>().job);
+                    return;
+                }
+            }
+            run_with_twin<P + 1>(pack, bx, by, bz, lds);
+        } else {
+            Job::run(pack.job, bx, by, bz, lds);
+        }
+    }
     // The block counts and grids of all the pack's jobs, read in one batch of scalar loads before the block knows which job is
     // its own (found one job after the other, each count would be a dependent load).
     __device__ __attribute__((always_inline)) static inline void header(const JobPack& pack, unsigned* blocks_of, unsigned* grid_x_of, unsigned* grid_y_of) {
@@ -2080,7 +2172,8 @@ struct JobPack<Job, Rest...> {
         if (block < blocks_of[I]) {
             const unsigned bx = block % grid_x_of[I];
             const unsigned q = block / grid_x_of[I];
-            Job::run(pack.job, bx, q % grid_y_of[I], q / grid_y_of[I], lds);
+            const unsigned by = q % grid_y_of[I], bz = q / grid_y_of[I];
+            run_with_twin<1>(pack, bx, by, bz, lds);
         } else {
             JobPack<Rest...>::template dispatch<I + 1>(pack.rest, block - blocks_of[I], blocks_of, grid_x_of, grid_y_of, lds);
         }

@@ -47,6 +47,11 @@ struct YuvView {
     int w, h;         // window size: the extent this plane produces
 };
 
+template <typename View>
+inline bool same_window(const View& a, const View& b) {
+    return a.data == b.data && a.pitch == b.pitch && a.img_w == b.img_w && a.img_h == b.img_h && a.ox == b.ox && a.oy == b.oy && a.w == b.w && a.h == b.h;
+}
+
 struct NoTail {};
 
 // SrcView: the window that is resampled (its w, h are the clamp limits); Pre: compute operations applied to each of

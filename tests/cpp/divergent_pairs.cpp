@@ -1,0 +1,111 @@
+// Divergent launches in which two chains read the same window of one image (their blocks are shared) beside chains that read other
+// windows, as user code: every chain's output is compared with the chain launched on its own, byte for byte.
+#include <fused_kernel/fused_kernel.h>
+
+#include <cstdio>
+#include <cstring>
+
+using namespace fk;
+
+static int failures = 0;
+
+template <typename T>
+static Ptr2D<T> image(uint w, uint h, uint seed, Stream& stream) {
+    Ptr2D<T> p(w, h);
+    for (uint y = 0; y < h; ++y)
+        for (uint x = 0; x < w; ++x) {
+            T v;
+            unsigned char* const b = reinterpret_cast<unsigned char*>(&v);
+            for (size_t i = 0; i < sizeof(T); ++i) b[i] = static_cast<unsigned char>((x * 31u + y * 17u + i * 101u) * seed >> 3);
+            p.at(x, y) = v;
+        }
+    p.upload(stream);
+    return p;
+}
+template <typename T>
+static void expect_same(Ptr2D<T>& a, Ptr2D<T>& b, Stream& stream, const char* what, uint w, uint h) {
+    a.download(stream);
+    b.download(stream);
+    stream.sync();
+    for (uint y = 0; y < a.dims().height; ++y)
+        for (uint x = 0; x < a.dims().width; ++x) {
+            const T p = a.at(x, y), q = b.at(x, y);
+            if (std::memcmp(&p, &q, sizeof(T)) != 0) {
+                std::printf("FAILED %s at %u,%u of %ux%u\n", what, x, y, w, h);
+                ++failures;
+                return;
+            }
+        }
+}
+template <typename Sequence>
+static void alone(Stream& stream, const Sequence& s) { executeOperations<TransformDPP<>>(stream, s.sender, s.receiver); }
+
+static void rgba(uint w, uint h, Stream& stream) {
+    const Ptr2D<uchar4> src = image<uchar4>(w, h, 7, stream);
+    const uint cw = w > 2 ? w - 2 : w, ch = h > 1 ? h - 1 : h;
+    Ptr2D<uchar> gray(w, h), gray1(w, h);
+    Ptr2D<uchar4> crop(cw, ch), crop1(cw, ch), whole(w, h), whole1(w, h);
+    Ptr2D<float3> bgr(w, h), bgr1(w, h);
+    const auto read = PerThreadRead<ND::_2D, uchar4>::build(src);
+    const auto to_gray = [&](Ptr2D<uchar>& o) { return buildOperationSequence(read, ColorConversion<ColorConversionCodes::COLOR_RGBA2GRAY, uchar4, uchar>::build(), PerThreadWrite<ND::_2D, uchar>::build(o)); };
+    const auto to_crop = [&](Ptr2D<uchar4>& o) { // another window of the same image: never shared
+        return buildOperationSequence(read.then(Crop<>::build(Rect(w > 2 ? 1u : 0u, h > 1 ? 1u : 0u, static_cast<int>(cw), static_cast<int>(ch)))), Mul<uchar4, int, int4>::build(2), SaturateCast<int4, uchar4>::build(),
+                                      PerThreadWrite<ND::_2D, uchar4>::build(o));
+    };
+    const auto to_bgr = [&](Ptr2D<float3>& o) {
+        return buildOperationSequence(read, ColorConversion<ColorConversionCodes::COLOR_RGBA2BGR, uchar4, uchar3>::build(), Cast<uchar3, float3>::build(), Sub<float3>::build(make_set<float3>(0.5f)),
+                                      PerThreadWrite<ND::_2D, float3>::build(o));
+    };
+    const auto to_whole = [&](Ptr2D<uchar4>& o) { return buildOperationSequence(read, Mul<uchar4, int, int4>::build(3), SaturateCast<int4, uchar4>::build(), PerThreadWrite<ND::_2D, uchar4>::build(o)); };
+    executeOperations<DivergentBatchTransformDPP<>>(stream, to_gray(gray), to_crop(crop), to_bgr(bgr), to_whole(whole));
+    alone(stream, to_gray(gray1));
+    alone(stream, to_crop(crop1));
+    alone(stream, to_bgr(bgr1));
+    alone(stream, to_whole(whole1));
+    expect_same(gray, gray1, stream, "gray", w, h);
+    expect_same(crop, crop1, stream, "crop", w, h);
+    expect_same(bgr, bgr1, stream, "bgr", w, h);
+    expect_same(whole, whole1, stream, "whole", w, h);
+}
+
+// float sources pass through LDS on their way in as well
+static void floats(uint w, uint h, Stream& stream) {
+    const Ptr2D<uchar3> bytes = image<uchar3>(w, h, 11, stream);
+    Ptr2D<float3> src(w, h), a(w, h), a1(w, h), b(w, h), b1(w, h);
+    executeOperations<TransformDPP<>>(stream, PerThreadRead<ND::_2D, uchar3>::build(bytes), Cast<uchar3, float3>::build(), PerThreadWrite<ND::_2D, float3>::build(src));
+    const auto read = PerThreadRead<ND::_2D, float3>::build(src);
+    const auto times = [&](float f, Ptr2D<float3>& o) { return buildOperationSequence(read, Mul<float3>::build(make_set<float3>(f)), PerThreadWrite<ND::_2D, float3>::build(o)); };
+    const auto plus = [&](float f, Ptr2D<float3>& o) { return buildOperationSequence(read, Add<float3>::build(make_set<float3>(f)), PerThreadWrite<ND::_2D, float3>::build(o)); };
+    executeOperations<DivergentBatchTransformDPP<>>(stream, times(1.5f, a), plus(2.5f, b));
+    alone(stream, times(1.5f, a1));
+    alone(stream, plus(2.5f, b1));
+    expect_same(a, a1, stream, "times", w, h);
+    expect_same(b, b1, stream, "plus", w, h);
+}
+
+static void nv12(uint w, uint h, Stream& stream) {
+    constexpr PixelFormat PF = PixelFormat::NV12;
+    const Ptr2D<uchar> raw = image<uchar>(w, h + h / 2, 5, stream);
+    const Image<PF> frame(raw, w, h);
+    Ptr2D<uchar3> yuv(w, h), yuv1(w, h), rgb(w, h), rgb1(w, h);
+    const auto unpack = [&](Ptr2D<uchar3>& o) { return buildOperationSequence(ReadYUV<PF>::build(frame), PerThreadWrite<ND::_2D, uchar3>::build(o)); };
+    const auto convert = [&](Ptr2D<uchar3>& o) {
+        return buildOperationSequence(ReadYUV<PF>::build(frame), ConvertYUVToRGB<PF, ColorRange::Full, ColorPrimitives::bt709, false>::build(), PerThreadWrite<ND::_2D, uchar3>::build(o));
+    };
+    executeOperations<DivergentBatchTransformDPP<>>(stream, unpack(yuv), convert(rgb));
+    alone(stream, unpack(yuv1));
+    alone(stream, convert(rgb1));
+    expect_same(yuv, yuv1, stream, "yuv", w, h);
+    expect_same(rgb, rgb1, stream, "rgb", w, h);
+}
+
+int main() {
+    Stream stream;
+    for (const auto& s : { std::pair<uint, uint>(1, 1), { 3, 3 }, { 61, 9 }, { 256, 4 }, { 257, 5 }, { 1030, 3 } }) {
+        rgba(s.first, s.second, stream);
+        floats(s.first, s.second, stream);
+        nv12(2 * s.first, 2 * s.second, stream);
+    }
+    if (failures == 0) std::printf("divergent_pairs ok\n");
+    return failures == 0 ? 0 : 1;
+}

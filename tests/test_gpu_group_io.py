@@ -84,3 +84,11 @@ def test_windows_at_odd_rows_and_columns_as_user_code():
     assert os.path.exists(exe), "tests/cpp/yuv_windows is not built"
     proc = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
     assert proc.returncode == 0 and "yuv_windows ok" in proc.stdout, proc.stdout
+
+
+def test_divergent_chains_over_one_window_as_user_code():
+    """Chains of a divergent launch that read the same window run in one set of blocks; beside them chains that do not."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "divergent_pairs")
+    assert os.path.exists(exe), "tests/cpp/divergent_pairs is not built"
+    proc = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert proc.returncode == 0 and "divergent_pairs ok" in proc.stdout, proc.stdout
