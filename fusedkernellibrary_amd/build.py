@@ -3,6 +3,7 @@
   libfk_hip_rt.so   the C runtime ABI of include/fk_hip_rt.h (csrc/fk_hip_rt.cpp)
   libfk_capi.so     the chain entry points of include/fk_capi.h (csrc/fk_capi*.hip), i.e. the
                     fused kernels instantiated from the fk:: templates under include/fk/
+  _fk_host.so       the Python side's marshalling (csrc/fk_host.cpp), a CPython extension that reads torch tensors
 
   benchmarks/reference_sweeps   the reference's benchmark sweeps (benchmarks/reference_sweeps.cpp), a program
 
@@ -67,6 +68,20 @@ def build_capi(extra_defines=(), name="libfk_capi.so"):
         objs = list(pool.map(compile_one, CAPI_SOURCES))
     _run([hipcc(), *objs, "--offload-arch=gfx950", "-fPIC", "-shared", "-L" + HERE, "-lfk_hip_rt", "-Wl,-rpath,$ORIGIN", "-o", out])
     shutil.rmtree(objdir, ignore_errors=True)
+    return out
+
+
+def build_host():
+    """The marshalling extension: host code only, against Python's and torch's headers."""
+    import sysconfig
+    import torch
+    home = os.path.dirname(torch.__file__)
+    out = os.path.join(HERE, "_fk_host.so")
+    _run([shutil.which("g++") or "g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi()), "-isystem", os.path.join(home, "include"), "-isystem",
+          os.path.join(home, "include", "torch", "csrc", "api", "include"), "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+          "-isystem", sysconfig.get_paths()["include"], "-I" + INCLUDE, os.path.join(CSRC, "fk_host.cpp"), "-L" + os.path.join(home, "lib"),
+          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-o", out])
     return out
 
 
@@ -164,7 +179,7 @@ def build_all():
     from concurrent.futures import ThreadPoolExecutor
     outs = [build_runtime()]  # the others link against it
     with ThreadPoolExecutor(max_workers=4) as pool:
-        jobs = [pool.submit(build_capi), pool.submit(build_literal_capi), pool.submit(build_cpp_tests), pool.submit(build_benchmarks),
+        jobs = [pool.submit(build_capi), pool.submit(build_literal_capi), pool.submit(build_host), pool.submit(build_cpp_tests), pool.submit(build_benchmarks),
                 pool.submit(build_reference_tests)]
         for job in jobs:
             res = job.result()

@@ -1,0 +1,618 @@
+// fk_host.cpp — the Python side's marshalling in native code: takes torch tensors, regions and values as Python objects, checks
+// them, and calls the chain entry points of include/fk_capi.h.  A CPython extension module (_fk_host) that the package's
+// __init__.py loads beside libfk_capi.so; it holds no kernel and makes no GPU call of its own.
+//
+// Why native: the calls of this library are a few microseconds of GPU work each, and building the same arguments in Python
+// (attribute by attribute, one ctypes object per region) cost 6-9 us per call and 90 us for a batch of fifty images.  Here a tensor's
+// pointer, sizes and strides are read from its C++ object, a region is four integers, and the arguments live on the stack.
+// A chain bound for a launch loop (defer) keeps its arguments by value and is called without any marshalling.
+//
+// The Python interpreter's lock is released around the library call, as ctypes does.
+#include <torch/csrc/autograd/python_variable.h>
+#include <c10/hip/HIPStream.h>
+
+#include <array>
+#include <functional>
+#include <string>
+#include <vector>
+
+#include "fk_capi.h"
+
+namespace {
+
+// ---- the entry points: addresses handed over by the package when it has loaded a variant of the library ------------------
+#define FK_CHAINS(X)                                                                                                                                          \
+    X(fk_crop_resize_muls_bgr_tensor) X(fk_crop_resize_muls_bgr_tensor_noalloc) X(fk_muladd_chain_f32c3) X(fk_single_op_f32c3)                                 \
+    X(fk_batch_crop_resize_norm_split) X(fk_resize_crop_tiles) X(fk_rgba2gray_u8c4) X(fk_resize_mul_u8c4_f32c4) X(fk_crop_mul_saturate_u8c4)                   \
+    X(fk_rgba2bgr_sub_u8c4_f32c3) X(fk_divergent4_u8c4) X(fk_batch_crop_cast_tensor) X(fk_batch_windows_saturate_muls_f32) X(fk_read_yuv) X(fk_write_yuv)      \
+    X(fk_yuv_to_rgb) X(fk_yuv_crop_resize_norm_split) X(fk_border_crop_u8c3) X(fk_warp_u8c3_f32c3) X(fk_deinterlace_u8c3_f32c3) X(fk_tensor_relayout_f32c3)    \
+    X(fk_circular_tensor_read_f32c3) X(fk_circular_tensor_update_u8c3_split_f32) X(fk_conditional_copy_u8c3) X(fk_conditional_resize_f32c3)                    \
+    X(fk_muladd_midwrite_f32c3) X(fk_batch_crop_cast_images) X(fk_tensor_mul_f32c3) X(fk_set_to_f32c3_tensor)
+
+struct Library {
+#define FK_MEMBER(name) decltype(&::name) name = nullptr;
+    FK_CHAINS(FK_MEMBER)
+#undef FK_MEMBER
+    decltype(&::fk_last_error) fk_last_error = nullptr;
+};
+Library lib;
+PyObject* fk_error = nullptr; // the package's FkError
+
+// ---- errors: a Python exception that has been set, thrown through C++ frames ----------------------------------------------
+struct PythonError {};
+[[noreturn]] void raise(PyObject* type, const char* text) {
+    PyErr_SetString(type, text);
+    throw PythonError{};
+}
+[[noreturn]] void fail(const char* text) { raise(fk_error, text); }
+void require(const bool condition, const char* text) {
+    if (!condition) raise(PyExc_AssertionError, text);
+}
+[[noreturn]] void fail_call(const int rc) {
+    const char* const kind = rc == FK_ERR_UNSUPPORTED ? "unsupported" : rc == FK_ERR_RUNTIME ? "runtime" : rc == FK_ERR_ARGUMENT ? "argument" : nullptr;
+    fail(("fk call failed (" + (kind != nullptr ? std::string(kind) : std::to_string(rc)) + "): " + lib.fk_last_error()).c_str());
+}
+
+// ---- Python values -------------------------------------------------------------------------------------------------------
+int to_int(PyObject* o) { // int(o)
+    if (PyLong_Check(o)) {
+        const long v = PyLong_AsLong(o);
+        if (v == -1 && PyErr_Occurred()) throw PythonError{};
+        return static_cast<int>(v);
+    }
+    PyObject* const n = PyNumber_Long(o);
+    if (n == nullptr) throw PythonError{};
+    const long v = PyLong_AsLong(n);
+    Py_DECREF(n);
+    if (v == -1 && PyErr_Occurred()) throw PythonError{};
+    return static_cast<int>(v);
+}
+float to_float(PyObject* o) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw PythonError{};
+    return static_cast<float>(v);
+}
+bool to_bool(PyObject* o) {
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw PythonError{};
+    return v != 0;
+}
+// the items of a list, tuple or any other iterable
+class Items {
+public:
+    explicit Items(PyObject* o) : fast(PySequence_Fast(o, "expected a sequence")) {
+        if (fast == nullptr) throw PythonError{};
+    }
+    ~Items() { Py_DECREF(fast); }
+    Items(const Items&) = delete;
+    Items& operator=(const Items&) = delete;
+    int size() const { return static_cast<int>(PySequence_Fast_GET_SIZE(fast)); }
+    PyObject* operator[](const int i) const { return PySequence_Fast_GET_ITEM(fast, i); }
+
+private:
+    PyObject* fast;
+};
+using Float3 = std::array<float, 3>;
+Float3 to_float3(PyObject* o) {
+    const Items v(o);
+    if (v.size() > 3) raise(PyExc_IndexError, "expected three values");
+    Float3 f{};
+    for (int i = 0; i < v.size(); ++i) f[static_cast<size_t>(i)] = to_float(v[i]);
+    return f;
+}
+using Byte3 = std::array<uint8_t, 3>;
+Byte3 to_byte3(PyObject* o) {
+    const Items v(o);
+    if (v.size() > 3) raise(PyExc_IndexError, "expected three values");
+    Byte3 b{};
+    for (int i = 0; i < v.size(); ++i) b[static_cast<size_t>(i)] = static_cast<uint8_t>(to_int(v[i]));
+    return b;
+}
+fk_rect to_rect(PyObject* o) {
+    const Items v(o);
+    if (v.size() > 4) raise(PyExc_TypeError, "a region is (x, y, width, height)");
+    int f[4] = { 0, 0, 0, 0 };
+    for (int i = 0; i < v.size(); ++i) f[i] = to_int(v[i]);
+    return fk_rect{ f[0], f[1], f[2], f[3] };
+}
+std::vector<fk_rect> to_rects(PyObject* o) {
+    const Items v(o);
+    std::vector<fk_rect> r;
+    r.reserve(static_cast<size_t>(v.size()));
+    for (int i = 0; i < v.size(); ++i) r.push_back(to_rect(v[i]));
+    return r;
+}
+void* to_stream(PyObject* o) {
+    if (o == Py_None) return c10::hip::getCurrentHIPStream().stream(); // the current stream of the current device
+    void* const s = PyLong_AsVoidPtr(o);
+    if (s == nullptr && PyErr_Occurred()) throw PythonError{};
+    return s;
+}
+
+// ---- tensors -------------------------------------------------------------------------------------------------------------
+const at::Tensor& to_tensor(PyObject* o) {
+    if (!THPVariable_Check(o)) raise(PyExc_TypeError, "expected a torch tensor");
+    return THPVariable_Unpack(o);
+}
+const at::Tensor& on_device(PyObject* o, const at::ScalarType type, const char* text) {
+    const at::Tensor& t = to_tensor(o);
+    if (!t.is_cuda()) fail("tensors must live on the GPU");
+    if (t.scalar_type() != type) fail(text);
+    const int64_t d = t.dim();
+    if (d < 1 || t.stride(d - 1) != 1 || (d >= 3 && t.stride(d - 2) != t.size(d - 1))) fail("pixels must be contiguous along a row");
+    return t;
+}
+const at::Tensor& bytes(PyObject* o) { return on_device(o, at::kByte, "expected a uint8 tensor"); }
+const at::Tensor& floats(PyObject* o) { return on_device(o, at::kFloat, "expected a float32 tensor"); }
+struct ImageArg {
+    void* data;
+    int w, h;
+    size_t pitch; // bytes
+    bool operator==(const ImageArg& o) const { return w == o.w && h == o.h && pitch == o.pitch; }
+};
+// (h, w, c) whose row stride is the pitch
+ImageArg image(const at::Tensor& t) {
+    if (t.dim() < 2) raise(PyExc_IndexError, "an image has rows and columns");
+    return { t.data_ptr(), static_cast<int>(t.size(1)), static_cast<int>(t.size(0)), static_cast<size_t>(t.stride(0)) * t.element_size() };
+}
+// several images of one size and pitch
+std::vector<void*> same_images(const Items& list, const at::Tensor& (*of)(PyObject*), ImageArg& first) {
+    if (list.size() == 0) raise(PyExc_IndexError, "no images");
+    std::vector<void*> data;
+    data.reserve(static_cast<size_t>(list.size()));
+    for (int i = 0; i < list.size(); ++i) {
+        const ImageArg im = image(of(list[i]));
+        if (i == 0) first = im;
+        require(im == first, "images of one size and pitch");
+        data.push_back(im.data);
+    }
+    return data;
+}
+// a contiguous result of n planes: (n, h, w, 3) or, planar, (n, 3, h, w)
+struct Planes {
+    float* data;
+    int n, w, h;
+};
+Planes packed_planes(PyObject* o) {
+    const at::Tensor& t = floats(o);
+    if (t.dim() != 4) raise(PyExc_ValueError, "expected a tensor of planes");
+    require(t.is_contiguous(), "the result must be contiguous");
+    return { static_cast<float*>(t.data_ptr()), static_cast<int>(t.size(0)), static_cast<int>(t.size(2)), static_cast<int>(t.size(1)) };
+}
+struct RawArg {
+    void* data;
+    size_t pitch;
+};
+bool wide_format(const int f) { return f == FK_PF_P010 || f == FK_PF_P210 || f == FK_PF_Y210; }
+RawArg raw_image(PyObject* o, const int format) {
+    const at::Tensor& t = to_tensor(o);
+    if (!t.is_cuda() || t.dim() != 2 || t.stride(1) != 1) fail("a raw YUV image is a 2D GPU tensor with contiguous rows");
+    const at::ScalarType s = t.scalar_type();
+    if (wide_format(format) ? (s != at::kUInt16 && s != at::kShort) : s != at::kByte) fail("raw YUV image has the wrong element type for its format");
+    return { t.data_ptr(), static_cast<size_t>(t.stride(0)) * t.element_size() };
+}
+const at::Tensor& pixels(PyObject* o) {
+    const at::Tensor& t = to_tensor(o);
+    if (!t.is_cuda() || t.dim() != 3 || t.stride(2) != 1 || t.stride(1) != t.size(2)) fail("pixels must be a (h, w, c) GPU tensor, contiguous along a row");
+    return t;
+}
+
+// ---- a chain with its arguments: called now, or kept and called in a loop -----------------------------------------------------
+struct Bound {
+    PyObject_HEAD
+    vectorcallfunc vectorcall;
+    std::function<int()>* call;
+};
+PyObject* bound_call(PyObject* self, PyObject* const*, const size_t nargsf, PyObject* kwnames) {
+    if (PyVectorcall_NARGS(nargsf) != 0 || (kwnames != nullptr && PyTuple_GET_SIZE(kwnames) != 0)) {
+        PyErr_SetString(PyExc_TypeError, "a bound chain takes no arguments");
+        return nullptr;
+    }
+    const std::function<int()>& call = *reinterpret_cast<Bound*>(self)->call;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = call();
+    Py_END_ALLOW_THREADS
+    if (rc == FK_OK) Py_RETURN_NONE;
+    try {
+        fail_call(rc);
+    } catch (const PythonError&) {
+    }
+    return nullptr;
+}
+void bound_dealloc(PyObject* self) {
+    delete reinterpret_cast<Bound*>(self)->call;
+    Py_TYPE(self)->tp_free(self);
+}
+PyTypeObject bound_type = { PyVarObject_HEAD_INIT(nullptr, 0) };
+
+// `call` holds everything the entry point needs by value
+template <typename Call>
+PyObject* now_or_deferred(PyObject* defer, PyObject* result, const Call& call) {
+    if (to_bool(defer)) {
+        Bound* const b = PyObject_New(Bound, &bound_type);
+        if (b == nullptr) throw PythonError{};
+        b->vectorcall = bound_call;
+        b->call = new std::function<int()>(call);
+        return reinterpret_cast<PyObject*>(b);
+    }
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = call();
+    Py_END_ALLOW_THREADS
+    if (rc != FK_OK) fail_call(rc);
+    Py_INCREF(result);
+    return result;
+}
+
+// ---- the chains: arguments in the order of the package's functions, all of them given --------------------------------------
+using Args = PyObject* const*;
+
+PyObject* readme(Args a, decltype(&::fk_crop_resize_muls_bgr_tensor) fn) { // src, rects, out, aspect, background, mul, sub, div, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    const Planes o = packed_planes(a[2]);
+    const std::vector<fk_rect> rects = to_rects(a[1]);
+    require(o.n == static_cast<int>(rects.size()), "one plane of the result per region");
+    const int aspect = to_int(a[3]);
+    const Float3 bg = to_float3(a[4]), mul = to_float3(a[5]), sub = to_float3(a[6]), div = to_float3(a[7]);
+    void* const stream = to_stream(a[8]);
+    return now_or_deferred(a[9], a[2], [=] {
+        return fn(s.data, s.w, s.h, s.pitch, rects.data(), o.n, o.w, o.h, aspect, bg.data(), mul.data(), sub.data(), div.data(), o.data, stream);
+    });
+}
+PyObject* crop_resize_muls_bgr_tensor(Args a) { return readme(a, lib.fk_crop_resize_muls_bgr_tensor); }
+PyObject* crop_resize_muls_bgr_tensor_noalloc(Args a) { return readme(a, lib.fk_crop_resize_muls_bgr_tensor_noalloc); }
+
+PyObject* muladd_chain_f32c3(Args a) { // src, dst, depth, mul_v, add_v, stream, defer
+    const ImageArg s = image(floats(a[0])), d = image(floats(a[1]));
+    require(s.w == d.w && s.h == d.h, "images of one size");
+    const int depth = to_int(a[2]);
+    const float mul = to_float(a[3]), add = to_float(a[4]);
+    void* const stream = to_stream(a[5]);
+    return now_or_deferred(a[6], a[1], [=, fn = lib.fk_muladd_chain_f32c3] { return fn(s.data, s.w, s.h, s.pitch, depth, mul, add, d.data, d.pitch, stream); });
+}
+PyObject* single_op_f32c3(Args a) { // src, dst, is_add, v, stream, defer
+    const ImageArg s = image(floats(a[0])), d = image(floats(a[1]));
+    require(s.w == d.w && s.h == d.h, "images of one size");
+    const int is_add = to_int(a[2]);
+    const float v = to_float(a[3]);
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[1], [=, fn = lib.fk_single_op_f32c3] { return fn(s.data, s.w, s.h, s.pitch, is_add, v, d.data, d.pitch, stream); });
+}
+PyObject* batch_crop_resize_norm_split(Args a) { // srcs, rects, out, div1, sub, div2, stream, defer
+    ImageArg s{};
+    const std::vector<void*> data = same_images(Items(a[0]), bytes, s);
+    const std::vector<fk_rect> rects = to_rects(a[1]);
+    const at::Tensor& out = floats(a[2]);
+    const int n = static_cast<int>(data.size());
+    require(out.dim() == 4 && out.size(0) == n && rects.size() == data.size() && out.size(1) == 3 && out.is_contiguous(), "out is (n, 3, h, w), contiguous, one plane per image and region");
+    const int w = static_cast<int>(out.size(3)), h = static_cast<int>(out.size(2));
+    float* const o = static_cast<float*>(out.data_ptr());
+    const Float3 d1 = to_float3(a[3]), sub = to_float3(a[4]), d2 = to_float3(a[5]);
+    void* const stream = to_stream(a[6]);
+    return now_or_deferred(a[7], a[2], [=, fn = lib.fk_batch_crop_resize_norm_split] {
+        return fn(data.data(), s.w, s.h, s.pitch, rects.data(), n, w, h, d1.data(), sub.data(), d2.data(), o, stream);
+    });
+}
+PyObject* resize_crop_tiles(Args a) { // src, resized, rects, out, mul, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    const Planes o = packed_planes(a[3]);
+    const std::vector<fk_rect> rects = to_rects(a[2]);
+    require(o.n == static_cast<int>(rects.size()), "one plane of the result per tile");
+    const Items resized(a[1]);
+    if (resized.size() < 2) raise(PyExc_IndexError, "resized is (width, height)");
+    const int rw = to_int(resized[0]), rh = to_int(resized[1]);
+    const Float3 mul = to_float3(a[4]);
+    void* const stream = to_stream(a[5]);
+    return now_or_deferred(a[6], a[3], [=, fn = lib.fk_resize_crop_tiles] { return fn(s.data, s.w, s.h, s.pitch, rw, rh, rects.data(), o.n, o.w, o.h, mul.data(), o.data, stream); });
+}
+PyObject* rgba2gray_u8c4(Args a) { // src, dst, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    const at::Tensor& d = bytes(a[1]);
+    void* const dst = d.data_ptr();
+    const size_t pitch = static_cast<size_t>(d.stride(0));
+    void* const stream = to_stream(a[2]);
+    return now_or_deferred(a[3], a[1], [=, fn = lib.fk_rgba2gray_u8c4] { return fn(s.data, s.w, s.h, s.pitch, dst, pitch, stream); });
+}
+PyObject* resize_mul_u8c4_f32c4(Args a) { // src, dst, mul_v, stream, defer
+    const ImageArg s = image(bytes(a[0])), d = image(floats(a[1]));
+    const float mul = to_float(a[2]);
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[1], [=, fn = lib.fk_resize_mul_u8c4_f32c4] { return fn(s.data, s.w, s.h, s.pitch, d.w, d.h, mul, d.data, d.pitch, stream); });
+}
+PyObject* crop_mul_saturate_u8c4(Args a) { // src, rect, dst, mul_v, stream, defer
+    const ImageArg s = image(bytes(a[0])), d = image(bytes(a[2]));
+    const fk_rect r = to_rect(a[1]);
+    const int mul = to_int(a[3]);
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[2], [=, fn = lib.fk_crop_mul_saturate_u8c4] { return fn(s.data, s.w, s.h, s.pitch, r, mul, d.data, d.pitch, stream); });
+}
+PyObject* rgba2bgr_sub_u8c4_f32c3(Args a) { // src, dst, sub_v, stream, defer
+    const ImageArg s = image(bytes(a[0])), d = image(floats(a[1]));
+    const float sub = to_float(a[2]);
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[1], [=, fn = lib.fk_rgba2bgr_sub_u8c4_f32c3] { return fn(s.data, s.w, s.h, s.pitch, sub, d.data, d.pitch, stream); });
+}
+PyObject* divergent4_u8c4(Args a) { // src, gray_out, resized_out, mul_b, rect_c, mul_c, crop_out, sub_d, bgr_out, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    for (const int i : { 1, 2, 6, 8 }) require(to_tensor(a[i]).is_contiguous(), "the results must be contiguous");
+    void* const gray = bytes(a[1]).data_ptr();
+    const ImageArg resized = image(floats(a[2]));
+    const float mul_b = to_float(a[3]), sub_d = to_float(a[7]);
+    const fk_rect r = to_rect(a[4]);
+    const int mul_c = to_int(a[5]);
+    void* const crop = bytes(a[6]).data_ptr();
+    void* const bgr = floats(a[8]).data_ptr();
+    void* const stream = to_stream(a[9]);
+    return now_or_deferred(a[10], Py_None, [=, fn = lib.fk_divergent4_u8c4] {
+        return fn(s.data, s.w, s.h, s.pitch, gray, resized.w, resized.h, mul_b, resized.data, r, mul_c, crop, sub_d, bgr, stream);
+    });
+}
+PyObject* batch_crop_cast_tensor(Args a) { // src, rects, out, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    const Planes o = packed_planes(a[2]);
+    const std::vector<fk_rect> rects = to_rects(a[1]);
+    require(o.n == static_cast<int>(rects.size()), "one plane of the result per region");
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[2], [=, fn = lib.fk_batch_crop_cast_tensor] { return fn(s.data, s.w, s.h, s.pitch, rects.data(), o.n, o.w, o.h, o.data, stream); });
+}
+PyObject* batch_windows_saturate_muls_f32(Args a) { // src, rects, out, mul_v, sub_v, div_v, stream, defer
+    const at::Tensor& src = bytes(a[0]);
+    if (src.dim() != 2) fail("expected a (h, w) image of bytes");
+    const ImageArg s = image(src);
+    const at::Tensor& out = floats(a[2]);
+    const std::vector<fk_rect> rects = to_rects(a[1]);
+    if (rects.empty()) raise(PyExc_IndexError, "no windows");
+    const int n = static_cast<int>(rects.size());
+    require(out.dim() == 3 && out.size(0) == n && out.size(1) == rects[0].height && out.size(2) == rects[0].width && out.is_contiguous(), "out is (n, height, width), contiguous");
+    float* const o = static_cast<float*>(out.data_ptr());
+    const float mul = to_float(a[3]), sub = to_float(a[4]), div = to_float(a[5]);
+    void* const stream = to_stream(a[6]);
+    return now_or_deferred(a[7], a[2], [=, fn = lib.fk_batch_windows_saturate_muls_f32] { return fn(s.data, s.w, s.h, s.pitch, rects.data(), n, mul, sub, div, o, stream); });
+}
+
+PyObject* read_yuv(Args a) { // fmt, raw, out, stream, defer
+    const int fmt = to_int(a[0]);
+    const RawArg raw = raw_image(a[1], fmt);
+    const ImageArg o = image(pixels(a[2]));
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[2], [=, fn = lib.fk_read_yuv] { return fn(fmt, raw.data, raw.pitch, o.w, o.h, o.data, o.pitch, stream); });
+}
+PyObject* write_yuv(Args a) { // fmt, pixels, raw, stream, defer
+    const int fmt = to_int(a[0]);
+    const ImageArg p = image(pixels(a[1]));
+    const RawArg raw = raw_image(a[2], fmt);
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[2], [=, fn = lib.fk_write_yuv] { return fn(fmt, p.data, p.pitch, p.w, p.h, raw.data, raw.pitch, stream); });
+}
+PyObject* yuv_to_rgb(Args a) { // fmt, color_range, primaries, raw, out, stream, defer
+    const int fmt = to_int(a[0]), range = to_int(a[1]), primaries = to_int(a[2]);
+    const RawArg raw = raw_image(a[3], fmt);
+    const at::Tensor& out = pixels(a[4]);
+    const ImageArg o = image(out);
+    const int64_t cn = out.size(2);
+    if (cn != 3 && cn != 4) fail("output pixels have 3 or 4 channels");
+    const int alpha = cn == 4 ? 1 : 0, float_out = out.scalar_type() == at::kFloat ? 1 : 0;
+    void* const stream = to_stream(a[5]);
+    return now_or_deferred(a[6], a[4], [=, fn = lib.fk_yuv_to_rgb] { return fn(fmt, range, primaries, alpha, float_out, raw.data, raw.pitch, o.w, o.h, o.data, o.pitch, stream); });
+}
+PyObject* yuv_crop_resize_norm_split(Args a) { // fmt, color_range, primaries, raw, size, crop, out, div_v, stream, defer
+    const int fmt = to_int(a[0]), range = to_int(a[1]), primaries = to_int(a[2]);
+    const RawArg raw = raw_image(a[3], fmt);
+    const Items size(a[4]);
+    if (size.size() < 2) raise(PyExc_IndexError, "size is (width, height)");
+    const int w = to_int(size[0]), h = to_int(size[1]);
+    const fk_rect crop = to_rect(a[5]);
+    const at::Tensor& out = floats(a[6]);
+    if (out.dim() != 3) raise(PyExc_ValueError, "out is (3, height, width)");
+    require(out.is_contiguous(), "the result must be contiguous");
+    const int dw = static_cast<int>(out.size(2)), dh = static_cast<int>(out.size(1));
+    float* const o = static_cast<float*>(out.data_ptr());
+    const float div = to_float(a[7]);
+    void* const stream = to_stream(a[8]);
+    return now_or_deferred(a[9], a[6], [=, fn = lib.fk_yuv_crop_resize_norm_split] { return fn(fmt, range, primaries, raw.data, raw.pitch, w, h, crop, dw, dh, div, o, stream); });
+}
+
+PyObject* border_crop_u8c3(Args a) { // border_type, src, left, top, out, value, stream, defer
+    const int type = to_int(a[0]), left = to_int(a[2]), top = to_int(a[3]);
+    const ImageArg s = image(bytes(a[1])), o = image(bytes(a[4]));
+    const Byte3 value = to_byte3(a[5]);
+    void* const stream = to_stream(a[6]);
+    return now_or_deferred(a[7], a[4], [=, fn = lib.fk_border_crop_u8c3] { return fn(type, s.data, s.w, s.h, s.pitch, left, top, o.w, o.h, value.data(), o.data, o.pitch, stream); });
+}
+PyObject* warp_u8c3_f32c3(Args a) { // warp_type, matrix, src, out, stream, defer
+    const int type = to_int(a[0]);
+    const ImageArg s = image(bytes(a[2])), o = image(floats(a[3]));
+    std::array<float, 9> m{}; // row-major, given flat or as rows
+    int given = 0;
+    const auto put = [&](PyObject* v) {
+        if (given >= 9) fail("matrix must be 2x3 (affine) or 3x3 (perspective)");
+        m[static_cast<size_t>(given++)] = to_float(v);
+    };
+    const Items rows(a[1]);
+    for (int i = 0; i < rows.size(); ++i) {
+        if (PyObject_HasAttrString(rows[i], "__len__")) {
+            const Items row(rows[i]);
+            for (int j = 0; j < row.size(); ++j) put(row[j]);
+        } else {
+            put(rows[i]);
+        }
+    }
+    if (given != (type == FK_WARP_AFFINE ? 6 : 9)) fail("matrix must be 2x3 (affine) or 3x3 (perspective)");
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[3], [=, fn = lib.fk_warp_u8c3_f32c3] { return fn(type, m.data(), s.data, s.w, s.h, s.pitch, o.w, o.h, o.data, o.pitch, stream); });
+}
+PyObject* deinterlace_u8c3_f32c3(Args a) { // kind, use_even_lines, src, out, stream, defer
+    const int kind = to_int(a[0]), even = to_int(a[1]);
+    const ImageArg s = image(bytes(a[2])), o = image(floats(a[3]));
+    require(s.w == o.w && s.h == o.h, "images of one size");
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[3], [=, fn = lib.fk_deinterlace_u8c3_f32c3] { return fn(kind, even, s.data, s.w, s.h, s.pitch, o.data, o.pitch, stream); });
+}
+
+PyObject* tensor_relayout_f32c3(Args a) { // mode, src, w, h, planes, out, stream, defer
+    const int mode = to_int(a[0]), w = to_int(a[2]), h = to_int(a[3]), planes = to_int(a[4]);
+    const at::Tensor &src = floats(a[1]), &out = floats(a[5]);
+    require(src.is_contiguous() && out.is_contiguous() && src.numel() == out.numel() && src.numel() == static_cast<int64_t>(planes) * h * w * 3, "contiguous tensors of planes * h * w * 3 elements");
+    const float* const s = static_cast<const float*>(src.data_ptr());
+    float* const o = static_cast<float*>(out.data_ptr());
+    void* const stream = to_stream(a[6]);
+    return now_or_deferred(a[7], a[5], [=, fn = lib.fk_tensor_relayout_f32c3] { return fn(mode, s, w, h, planes, o, stream); });
+}
+PyObject* circular_tensor_read_f32c3(Args a) { // direction, first, ring, out, stream, defer
+    const int direction = to_int(a[0]), first = to_int(a[1]);
+    const Planes r = packed_planes(a[2]), o = packed_planes(a[3]);
+    require(to_tensor(a[2]).sizes() == to_tensor(a[3]).sizes(), "tensors of one shape");
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[3], [=, fn = lib.fk_circular_tensor_read_f32c3] { return fn(direction, first, r.data, r.w, r.h, r.n, o.data, stream); });
+}
+PyObject* circular_tensor_update_u8c3_split_f32(Args a) { // frame, mul_v, tensor, ring, next_index, newest_first, stream, defer
+    const ImageArg f = image(bytes(a[0]));
+    const float mul = to_float(a[1]);
+    const at::Tensor &tensor = floats(a[2]), &ring = floats(a[3]);
+    const auto fits = [&](const at::Tensor& t) { return t.dim() == 4 && t.is_contiguous() && t.size(0) == tensor.size(0) && t.size(1) == 3 && t.size(2) == f.h && t.size(3) == f.w; };
+    require(fits(tensor) && fits(ring), "tensor and ring are (batch, 3, h, w), contiguous");
+    const int batch = static_cast<int>(tensor.size(0)), next = to_int(a[4]), newest = to_int(a[5]);
+    float *const t = static_cast<float*>(tensor.data_ptr()), *const r = static_cast<float*>(ring.data_ptr());
+    void* const stream = to_stream(a[6]);
+    PyObject* const done = now_or_deferred(a[7], Py_None, [=, fn = lib.fk_circular_tensor_update_u8c3_split_f32] { return fn(f.data, f.w, f.h, f.pitch, mul, t, r, batch, next, newest, stream); });
+    if (done != Py_None) return done; // (deferred)
+    Py_DECREF(done);
+    return PyLong_FromLong((next + 1) % batch); // the ring slot for the next update
+}
+
+PyObject* conditional_copy_u8c3(Args a) { // srcs, used, default, out, stream, defer
+    ImageArg s{};
+    const std::vector<void*> data = same_images(Items(a[0]), bytes, s);
+    const at::Tensor& out = bytes(a[3]);
+    const int n = static_cast<int>(data.size()), used = to_int(a[1]);
+    require(out.dim() == 4 && out.size(0) == n && out.size(1) == s.h && out.size(2) == s.w && out.size(3) == 3 && out.is_contiguous(), "out is (n, h, w, 3), contiguous");
+    void* const o = out.data_ptr();
+    const Byte3 d = to_byte3(a[2]);
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[3], [=, fn = lib.fk_conditional_copy_u8c3] { return fn(data.data(), s.w, s.h, s.pitch, n, used, d.data(), o, stream); });
+}
+PyObject* conditional_resize_f32c3(Args a) { // srcs, used, default, out, stream, defer
+    ImageArg s{};
+    const std::vector<void*> data = same_images(Items(a[0]), bytes, s);
+    const Planes o = packed_planes(a[3]);
+    const int n = static_cast<int>(data.size()), used = to_int(a[1]);
+    require(o.n == n && to_tensor(a[3]).size(3) == 3, "out is (n, dst_h, dst_w, 3), contiguous");
+    const Float3 d = to_float3(a[2]);
+    void* const stream = to_stream(a[4]);
+    return now_or_deferred(a[5], a[3], [=, fn = lib.fk_conditional_resize_f32c3] { return fn(data.data(), s.w, s.h, s.pitch, n, used, d.data(), o.w, o.h, o.data, stream); });
+}
+PyObject* muladd_midwrite_f32c3(Args a) { // src, mul_v, add_v, mid, out, stream, defer
+    const ImageArg s = image(floats(a[0])), m = image(floats(a[3])), o = image(floats(a[4]));
+    require(s.w == m.w && s.h == m.h && s.w == o.w && s.h == o.h, "images of one size");
+    const float mul = to_float(a[1]), add = to_float(a[2]);
+    void* const stream = to_stream(a[5]);
+    PyObject* const done = now_or_deferred(a[6], Py_None, [=, fn = lib.fk_muladd_midwrite_f32c3] { return fn(s.data, s.w, s.h, s.pitch, mul, add, m.data, m.pitch, o.data, o.pitch, stream); });
+    if (done != Py_None) return done; // (deferred)
+    Py_DECREF(done);
+    return PyTuple_Pack(2, a[3], a[4]);
+}
+PyObject* batch_crop_cast_images(Args a) { // src, rects, outs, stream, defer
+    const ImageArg s = image(bytes(a[0]));
+    ImageArg o{};
+    const std::vector<void*> data = same_images(Items(a[2]), floats, o);
+    const std::vector<fk_rect> rects = to_rects(a[1]);
+    require(data.size() == rects.size(), "one image per region");
+    const int n = static_cast<int>(rects.size());
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[2], [=, fn = lib.fk_batch_crop_cast_images] {
+        return fn(s.data, s.w, s.h, s.pitch, rects.data(), n, reinterpret_cast<float* const*>(data.data()), o.pitch, stream);
+    });
+}
+PyObject* tensor_mul_f32c3(Args a) { // src, mul, out, stream, defer
+    const Planes s = packed_planes(a[0]), o = packed_planes(a[2]);
+    require(to_tensor(a[0]).sizes() == to_tensor(a[2]).sizes() && to_tensor(a[0]).size(3) == 3, "(planes, h, w, 3) tensors of one shape");
+    const Float3 mul = to_float3(a[1]);
+    void* const stream = to_stream(a[3]);
+    return now_or_deferred(a[4], a[2], [=, fn = lib.fk_tensor_mul_f32c3] { return fn(s.data, s.w, s.h, s.n, mul.data(), o.data, stream); });
+}
+PyObject* set_to_f32c3_tensor(Args a) { // value, out, stream, defer
+    const at::Tensor& out = floats(a[1]);
+    require(out.dim() == 4 && out.size(3) == 3 && out.is_contiguous(), "out is (planes, h, w, 3), contiguous");
+    const Planes o = packed_planes(a[1]);
+    const Float3 value = to_float3(a[0]);
+    void* const stream = to_stream(a[2]);
+    return now_or_deferred(a[3], a[1], [=, fn = lib.fk_set_to_f32c3_tensor] { return fn(value.data(), o.data, o.w, o.h, o.n, stream); });
+}
+
+// ---- the module ------------------------------------------------------------------------------------------------------------
+template <PyObject* (*CHAIN)(Args), int COUNT>
+PyObject* entry(PyObject*, PyObject* const* args, const Py_ssize_t nargs) {
+    if (nargs != COUNT) {
+        PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", COUNT, nargs);
+        return nullptr;
+    }
+    if (lib.fk_last_error == nullptr) {
+        PyErr_SetString(PyExc_RuntimeError, "the chain library has not been bound");
+        return nullptr;
+    }
+    try {
+        return CHAIN(args);
+    } catch (const PythonError&) {
+        return nullptr;
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+}
+
+// bind({name: address}, FkError): the entry points of the loaded library
+PyObject* bind(PyObject*, PyObject* const* args, const Py_ssize_t nargs) {
+    if (nargs != 2 || !PyDict_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "bind(addresses, error type)");
+        return nullptr;
+    }
+    Library found;
+    const auto take = [&](const char* name, auto& to) {
+        PyObject* const v = PyDict_GetItemString(args[0], name);
+        void* const p = v != nullptr ? PyLong_AsVoidPtr(v) : nullptr;
+        if (p == nullptr) {
+            if (!PyErr_Occurred()) PyErr_Format(PyExc_KeyError, "no address for %s", name);
+            return false;
+        }
+        to = reinterpret_cast<std::decay_t<decltype(to)>>(p);
+        return true;
+    };
+#define FK_TAKE(name) if (!take(#name, found.name)) return nullptr;
+    FK_CHAINS(FK_TAKE)
+#undef FK_TAKE
+    if (!take("fk_last_error", found.fk_last_error)) return nullptr;
+    Py_INCREF(args[1]);
+    Py_XDECREF(fk_error);
+    fk_error = args[1];
+    lib = found;
+    Py_RETURN_NONE;
+}
+
+#define FK_METHOD(name, count) { #name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(entry<name, count>)), METH_FASTCALL, nullptr }
+PyMethodDef methods[] = {
+    { "bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL, nullptr },
+    FK_METHOD(crop_resize_muls_bgr_tensor, 10), FK_METHOD(crop_resize_muls_bgr_tensor_noalloc, 10), FK_METHOD(muladd_chain_f32c3, 7), FK_METHOD(single_op_f32c3, 6),
+    FK_METHOD(batch_crop_resize_norm_split, 8), FK_METHOD(resize_crop_tiles, 7), FK_METHOD(rgba2gray_u8c4, 4), FK_METHOD(resize_mul_u8c4_f32c4, 5),
+    FK_METHOD(crop_mul_saturate_u8c4, 6), FK_METHOD(rgba2bgr_sub_u8c4_f32c3, 5), FK_METHOD(divergent4_u8c4, 11), FK_METHOD(batch_crop_cast_tensor, 5),
+    FK_METHOD(batch_windows_saturate_muls_f32, 8), FK_METHOD(read_yuv, 5), FK_METHOD(write_yuv, 5), FK_METHOD(yuv_to_rgb, 7), FK_METHOD(yuv_crop_resize_norm_split, 10),
+    FK_METHOD(border_crop_u8c3, 8), FK_METHOD(warp_u8c3_f32c3, 6), FK_METHOD(deinterlace_u8c3_f32c3, 6), FK_METHOD(tensor_relayout_f32c3, 8),
+    FK_METHOD(circular_tensor_read_f32c3, 6), FK_METHOD(circular_tensor_update_u8c3_split_f32, 8), FK_METHOD(conditional_copy_u8c3, 6),
+    FK_METHOD(conditional_resize_f32c3, 6), FK_METHOD(muladd_midwrite_f32c3, 7), FK_METHOD(batch_crop_cast_images, 5), FK_METHOD(tensor_mul_f32c3, 5),
+    FK_METHOD(set_to_f32c3_tensor, 4), { nullptr, nullptr, 0, nullptr }
+};
+PyModuleDef module_def = { PyModuleDef_HEAD_INIT, "_fk_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr };
+
+} // namespace
+
+PyMODINIT_FUNC PyInit__fk_host(void) {
+    bound_type.tp_name = "fusedkernellibrary_amd.BoundChain";
+    bound_type.tp_basicsize = sizeof(Bound);
+    bound_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
+    bound_type.tp_doc = "a chain with its arguments; calling it enqueues it";
+    bound_type.tp_dealloc = bound_dealloc;
+    bound_type.tp_call = PyVectorcall_Call;
+    bound_type.tp_vectorcall_offset = offsetof(Bound, vectorcall);
+    if (PyType_Ready(&bound_type) < 0) return nullptr;
+    return PyModule_Create(&module_def);
+}

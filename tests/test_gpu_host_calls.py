@@ -1,0 +1,115 @@
+"""How the Python functions take their arguments: regions and values of any sequence type, the current or a given stream, bound
+calls, several threads, and errors before anything is enqueued.  Results against the CPU oracle, bit for bit."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import same_bits
+from oracle import binding as B
+
+pytestmark = pytest.mark.gpu
+RECTS = [(0, 0, 34, 25), (10, 10, 70, 15), (20, 20, 60, 59), (30, 30, 20, 23), (40, 40, 12, 11)]
+VALUES = (B.PRESERVE_AR, (0, 0, 0), (1.4,) * 3, (0.5,) * 3, (255.,) * 3)
+
+
+@pytest.fixture(scope="module")
+def case(oracle):
+    src = oracle.bytes(11, (128, 160, 3))
+    return torch.from_numpy(src).cuda(), oracle.crop_resize_muls_bgr_tensor(src, RECTS, (60, 60), *VALUES)
+
+
+@pytest.mark.parametrize("rects,values", [
+    (RECTS, VALUES), (tuple(map(list, RECTS)), (0, [0, 0, 0], [1.4] * 3, np.full(3, 0.5), np.full(3, 255))),
+    (np.array(RECTS), (np.int64(0), np.zeros(3), (np.float64(1.4),) * 3, (0.5, 0.5, 0.5), (255, 255, 255))),
+    ([[float(v) for v in r] for r in RECTS], VALUES)])
+def test_sequences_of_any_type(fk, case, rects, values):
+    src, want = case
+    out = torch.full((5, 60, 60, 3), float("nan"), device="cuda")
+    assert fk.crop_resize_muls_bgr_tensor(src, rects, out, *values) is out
+    assert same_bits(out.cpu().numpy(), want)
+    out.fill_(float("nan"))
+    bound = fk.crop_resize_muls_bgr_tensor(src, rects, out, *values, defer=True)
+    del rects, values  # what was bound does not depend on them
+    for _ in range(3):
+        out.fill_(float("nan"))
+        assert bound() is None
+        assert same_bits(out.cpu().numpy(), want)
+
+
+def test_streams(fk, case):
+    """A chain is enqueued behind what its stream already holds: each result is first overwritten there, late."""
+    src, want = case
+    side, given = torch.cuda.Stream(), torch.cuda.Stream()
+    outs = [torch.empty((5, 60, 60, 3), device="cuda") for _ in range(3)]
+    delay = torch.empty(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+
+    def occupy(stream, out):
+        with torch.cuda.stream(stream):
+            for _ in range(10):
+                delay.fill_(1.0)
+            out.fill_(float("nan"))
+
+    occupy(side, outs[0])
+    with torch.cuda.stream(side):
+        fk.crop_resize_muls_bgr_tensor(src, RECTS, outs[0], *VALUES)
+    side.synchronize()
+    assert same_bits(outs[0].cpu().numpy(), want)
+    occupy(given, outs[1])
+    with torch.cuda.stream(side):
+        fk.crop_resize_muls_bgr_tensor(src, RECTS, outs[1], *VALUES, stream=given.cuda_stream)
+    given.synchronize()
+    assert same_bits(outs[1].cpu().numpy(), want)
+    bound = fk.crop_resize_muls_bgr_tensor(src, RECTS, outs[2], *VALUES, stream=given.cuda_stream, defer=True)
+    occupy(given, outs[2])
+    bound()
+    given.synchronize()
+    assert same_bits(outs[2].cpu().numpy(), want)
+
+
+def test_threads(fk, oracle):
+    src = oracle.bytes(12, (200, 300, 3))
+    d = torch.from_numpy(src).cuda()
+    bad = []
+
+    def work(k):
+        rects = [(k + i, 2 * i, 40 + k, 30 + i) for i in range(1 + 3 * k)]
+        want = oracle.crop_resize_muls_bgr_tensor(src, rects, (33, 21), *VALUES)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            out = torch.empty((len(rects), 21, 33, 3), device="cuda")
+            bound = fk.crop_resize_muls_bgr_tensor(d, rects, out, *VALUES, defer=True)
+            for i in range(40):
+                if i % 2:
+                    bound()
+                else:
+                    fk.crop_resize_muls_bgr_tensor(d, rects, out, *VALUES)
+            torch.cuda.current_stream().synchronize()
+            if not same_bits(out.cpu().numpy(), want):
+                bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_refusals(fk, case):
+    src, _ = case
+    out = torch.empty((5, 60, 60, 3), device="cuda")
+    for bad, error in [((src.cpu(), RECTS, out), fk.FkError), ((src.float(), RECTS, out), fk.FkError), ((src, RECTS, out.double()), fk.FkError),
+                       ((src[:, ::2], RECTS, out), fk.FkError), ((src, RECTS[:4], out), AssertionError), ((src, RECTS, out.transpose(1, 2)), (AssertionError, fk.FkError)),
+                       ((src, [(0, 0, 400, 20)] * 5, out), fk.FkError), ((src, [(0, 0, 4, 20, 1)] * 5, out), TypeError), ((7, RECTS, out), TypeError),
+                       ((src, ["abcd"] * 5, out), ValueError)]:
+        with pytest.raises(error):
+            fk.crop_resize_muls_bgr_tensor(*bad, *VALUES)
+    with pytest.raises(TypeError):
+        fk.crop_resize_muls_bgr_tensor(src, RECTS, out, 0, (0, 0, 0), (1.4, "x", 1.4), (0.5,) * 3, (255.,) * 3)
+    with pytest.raises(fk.FkError, match="matrix"):
+        fk.warp_u8c3_f32c3(fk.WARP_AFFINE, [1, 0, 0], src, torch.empty((8, 8, 3), device="cuda"))
+    bound = fk.crop_resize_muls_bgr_tensor(src, [(0, 0, 400, 20)] * 5, out, *VALUES, defer=True)
+    with pytest.raises(fk.FkError, match="outside"):
+        bound()
