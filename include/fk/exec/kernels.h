@@ -68,6 +68,43 @@ __device__ __attribute__((always_inline)) inline void stream_store_at(const __am
 __device__ __attribute__((always_inline)) inline __amdgpu_buffer_rsrc_t image_buffer(const void* wave_uniform_base, const unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wave_uniform_base), 0, static_cast<int>(bytes), 0x00020000);
 }
+// ND dwords of an image's row, from the byte `at` of its descriptor on.  ANY: `at` need not be a multiple of four: the aligned
+// dwords that cover the run are fetched, one more than it has, and the run is shifted out of them when it is used (an unaligned
+// access would have to reach past the image's last bytes to return them: a dword that reaches past the range comes back as zero).
+// Down-scaled tiles of images with rows of 3 * w bytes, w not a multiple of four, were gathered from memory three bytes per tap
+// before (the bound: one request per byte and lane): eighteen 340x340 tiles of 1682x1126 seen at 1222x818 14.3 -> 10.7 us, 23 regions
+// of a 1366x768 frame to 299x299 12.3 -> 10.5 us; with whole-dword rows the same kernel is unchanged (24.8 us for five 1080p crops).
+template <int ND, bool ANY>
+struct QuadRun {
+    unsigned int w[ND + (ANY ? 1 : 0)];
+    unsigned int at;
+    __device__ __attribute__((always_inline)) inline void load(const __amdgpu_buffer_rsrc_t image, const unsigned from) {
+        constexpr int N = ND + (ANY ? 1 : 0);
+        static_assert(N >= 1 && N <= 5, "one to five dwords");
+        at = from;
+        const unsigned first = ANY ? from & ~3u : from;
+        if constexpr (N == 1) {
+            w[0] = __builtin_amdgcn_raw_buffer_load_b32(image, first, 0, 0);
+        } else if constexpr (N == 2) {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(image, first, 0, 0);
+            w[0] = v.x; w[1] = v.y;
+        } else if constexpr (N == 3) {
+            const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(image, first, 0, 0);
+            w[0] = v.x; w[1] = v.y; w[2] = v.z;
+        } else {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(image, first, 0, 0);
+            w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+            if constexpr (N == 5) w[4] = __builtin_amdgcn_raw_buffer_load_b32(image, first + 16u, 0, 0);
+        }
+    }
+    __device__ __attribute__((always_inline)) inline void take(unsigned int* out) const {
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            if constexpr (ANY) out[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], at & 3u);
+            else out[i] = w[i];
+        }
+    }
+};
 // the same address in every lane, for the compiler to see
 __device__ __attribute__((always_inline)) inline char* wave_uniform(char* p) {
     const size_t a = reinterpret_cast<size_t>(p);
@@ -483,35 +520,46 @@ struct SourceAccess<PlainView<T>> {
         const size_t first = reinterpret_cast<size_t>(v.data) + static_cast<size_t>(v.oy) * v.pitch + static_cast<size_t>(v.ox) * sizeof(T);
         return first % chunk == 0 && (v.h == 1 || v.pitch % chunk == 0);
     }
-    // ---- quads: pixels 4q .. 4q + 3 of a row of the PARENT image, fetched as the whole dwords they occupy ----
-    // Three-byte pixels: a quad is twelve bytes, three dwords, when the image starts at a whole dword and its rows are a
-    // whole number of dwords apart.
+    // ---- quads: pixels 4q .. 4q + 3 of a row of the PARENT image, fetched as the dwords they occupy ----
+    // Three-byte pixels: a quad is twelve bytes, three dwords when the image starts at a whole dword and its rows are a
+    // whole number of dwords apart (quads_aligned), and three dwords shifted out of four otherwise (ANY).
     static constexpr bool HAS_QUADS = sizeof(T) == 3 && alignof(T) == 1;
-    using Quad = dev::u32x3;
-    // bytes of the parent image from its first pixel to its last, up to the end of the last dword that holds one of them
+    template <bool ANY>
+    using RawQuad = dev::QuadRun<3, ANY>;
+    // bytes of the parent image from the dword that holds its first byte to the end of the last dword that holds one of its bytes
     static size_t quad_extent(const View& v) {
-        return ((static_cast<size_t>(v.img_h) - 1u) * v.pitch + static_cast<size_t>(v.img_w) * sizeof(T) + 3u) & ~static_cast<size_t>(3);
+        return ((reinterpret_cast<size_t>(v.data) & 3u) + (static_cast<size_t>(v.img_h) - 1u) * v.pitch + static_cast<size_t>(v.img_w) * sizeof(T) + 3u) & ~static_cast<size_t>(3);
     }
-    static bool quads_aligned(const View& v) { return reinterpret_cast<size_t>(v.data) % 4 == 0 && v.pitch % 4 == 0; }
+    __host__ __device__ __attribute__((always_inline)) static inline bool quads_aligned(const View& v) {
+        return ((static_cast<unsigned>(reinterpret_cast<size_t>(v.data)) | static_cast<unsigned>(v.pitch)) & 3u) == 0u;
+    }
     __device__ __attribute__((always_inline)) static inline __amdgpu_buffer_rsrc_t quad_buffer(const View& v) {
-        const unsigned bytes = ((static_cast<unsigned>(v.img_h) - 1u) * v.pitch + static_cast<unsigned>(v.img_w) * static_cast<unsigned>(sizeof(T)) + 3u) & ~3u;
-        return dev::image_buffer(v.data, bytes);
+        const unsigned start = static_cast<unsigned>(reinterpret_cast<size_t>(v.data)) & 3u;
+        const unsigned bytes = (start + (static_cast<unsigned>(v.img_h) - 1u) * v.pitch + static_cast<unsigned>(v.img_w) * static_cast<unsigned>(sizeof(T)) + 3u) & ~3u;
+        return dev::image_buffer(reinterpret_cast<const char*>(v.data) - start, bytes);
     }
-    __device__ __attribute__((always_inline)) static inline Quad load_quad(const __amdgpu_buffer_rsrc_t image, const View& v, const int q, const int py) {
-        return __builtin_amdgcn_raw_buffer_load_b96(image, static_cast<unsigned>(py) * v.pitch + static_cast<unsigned>(q) * 12u, 0, 0);
+    template <bool ANY>
+    __device__ __attribute__((always_inline)) static inline void load_quad(const __amdgpu_buffer_rsrc_t image, const View& v, const int q, const int py, RawQuad<ANY>& out) {
+        const unsigned start = ANY ? static_cast<unsigned>(reinterpret_cast<size_t>(v.data)) & 3u : 0u;
+        out.load(image, start + static_cast<unsigned>(py) * v.pitch + static_cast<unsigned>(q) * 12u);
     }
     // the four pixels, each in the low three bytes of a dword
-    __device__ __attribute__((always_inline)) static inline void quad_dwords(const Quad& w, unsigned int* px) {
-        px[0] = w.x;
-        px[1] = __builtin_amdgcn_alignbyte(w.y, w.x, 3u);
-        px[2] = __builtin_amdgcn_alignbyte(w.z, w.y, 2u);
-        px[3] = w.z >> 8u;
+    template <bool ANY>
+    __device__ __attribute__((always_inline)) static inline void quad_dwords(const RawQuad<ANY>& raw, unsigned int* px) {
+        unsigned int w[3];
+        raw.take(w);
+        px[0] = w[0];
+        px[1] = __builtin_amdgcn_alignbyte(w[1], w[0], 3u);
+        px[2] = __builtin_amdgcn_alignbyte(w[2], w[1], 2u);
+        px[3] = w[2] >> 8u;
     }
     // the four pixels as their type, each channel taken from the byte of the dword that holds it (a conversion to float
     // that follows is then one instruction per channel)
-    __device__ __attribute__((always_inline)) static inline void quad_pixels(const Quad& w, T* px) {
+    template <bool ANY>
+    __device__ __attribute__((always_inline)) static inline void quad_pixels(const RawQuad<ANY>& raw, T* px) {
         using B = VBase<T>;
-        const unsigned int d[3] = { w.x, w.y, w.z };
+        unsigned int d[3];
+        raw.take(d);
         const auto channel = [&](const int byte) { return static_cast<B>(static_cast<unsigned char>(d[byte >> 2] >> (8 * (byte & 3)))); };
 #pragma unroll
         for (int k = 0; k < 4; ++k) px[k] = T{ channel(3 * k), channel(3 * k + 1), channel(3 * k + 2) };
@@ -636,19 +684,22 @@ struct SourceAccess<YuvView<PF>> {
         else return true;
     }
     static constexpr bool HAS_QUADS = quads_supported();
-    using Quad = dev::u32x2;
+    template <bool ANY>
+    using RawQuad = dev::u32x2;
     static constexpr unsigned rows_of(const unsigned img_h) { return Layout::semi_planar ? img_h + ((img_h + 1u) >> 1) : img_h; }
     static constexpr unsigned row_bytes_of(const unsigned img_w) { return Layout::semi_planar ? ((img_w + 1u) & ~1u) : 2u * ((img_w + 1u) & ~1u); }
     static size_t quad_extent(const View& v) {
         return ((static_cast<size_t>(rows_of(static_cast<unsigned>(v.img_h))) - 1u) * v.pitch + row_bytes_of(static_cast<unsigned>(v.img_w)) + 3u) & ~static_cast<size_t>(3);
     }
-    static bool quads_aligned(const View& v) { return reinterpret_cast<size_t>(v.data) % 4 == 0 && v.pitch % 4 == 0; }
+    __host__ __device__ __attribute__((always_inline)) static inline bool quads_aligned(const View& v) {
+        return ((static_cast<unsigned>(reinterpret_cast<size_t>(v.data)) | static_cast<unsigned>(v.pitch)) & 3u) == 0u;
+    }
     __device__ __attribute__((always_inline)) static inline __amdgpu_buffer_rsrc_t quad_buffer(const View& v) {
         const unsigned bytes = ((rows_of(static_cast<unsigned>(v.img_h)) - 1u) * v.pitch + row_bytes_of(static_cast<unsigned>(v.img_w)) + 3u) & ~3u;
         return dev::image_buffer(v.data, bytes);
     }
-    __device__ __attribute__((always_inline)) static inline Quad load_quad(const __amdgpu_buffer_rsrc_t image, const View& v, const int q, const int py) {
-        Quad w;
+    template <bool ANY>
+    __device__ __attribute__((always_inline)) static inline void load_quad(const __amdgpu_buffer_rsrc_t image, const View& v, const int q, const int py, dev::u32x2& w) {
         if constexpr (Layout::semi_planar) {
             const unsigned at = static_cast<unsigned>(q) * 4u;
             w.x = __builtin_amdgcn_raw_buffer_load_b32(image, static_cast<unsigned>(py) * v.pitch + at, 0, 0);
@@ -656,11 +707,11 @@ struct SourceAccess<YuvView<PF>> {
         } else {
             w = __builtin_amdgcn_raw_buffer_load_b64(image, static_cast<unsigned>(py) * v.pitch + static_cast<unsigned>(q) * 8u, 0, 0);
         }
-        return w;
     }
     // the four {Y, U, V} pixels; the two pixels of a pair receive the very same chroma values, so that what is computed from
     // the chroma alone (centring, products with the matrix) is computed once per pair
-    __device__ __attribute__((always_inline)) static inline void quad_pixels(const Quad& w, Pixel* px) {
+    template <bool ANY>
+    __device__ __attribute__((always_inline)) static inline void quad_pixels(const dev::u32x2& w, Pixel* px) {
         if constexpr (Layout::semi_planar) {
             const Base cu[2] = { static_cast<Base>(w.y >> (8 * Layout::u)), static_cast<Base>(w.y >> (16 + 8 * Layout::u)) };
             const Base cv[2] = { static_cast<Base>(w.y >> (8 * Layout::v)), static_cast<Base>(w.y >> (16 + 8 * Layout::v)) };
@@ -1046,8 +1097,11 @@ __device__ __attribute__((always_inline)) inline T slot_to_pixel(const PixelSlot
 // One pixel from memory at any byte alignment, as whole dwords.  `row` points at byte 0 of the window row, `off` is the
 // pixel's byte offset in it; [valid_lo, valid_hi) are the byte offsets of that row that belong to the parent image, so
 // dwords that would reach past them are assembled from single bytes.
+// Three-byte pixels are fetched as one dword, [p, p + 4) for a p at a whole dword and [p - 1, p + 3) otherwise: its one byte that
+// is not the pixel's lies in an aligned dword that also holds a byte of the pixel, so the load cannot fault and needs no branch
+// (the loads of several rows are in flight together).
 // The dword at byte `voff` from `row - 1`, for a `row` that is the same for the whole wave: the address stays in scalar
-// registers and the lane adds its 32-bit offset.
+// registers and the lane adds its 32-bit offset, from row - 1 so that it is never negative.
 __device__ __attribute__((always_inline)) inline unsigned int load_dword_from_row(const char* row, unsigned voff) {
     struct __attribute__((packed)) UnalignedDword { unsigned int v; };
     using GlobalBytes = const __attribute__((address_space(1))) char*;
@@ -1065,14 +1119,6 @@ __device__ __attribute__((always_inline)) inline PixelSlot<T> load_pixel_slot(co
         const unsigned int* const p = reinterpret_cast<const unsigned int*>(row + off);
 #pragma unroll
         for (int i = 0; i < ND; ++i) s.w[i] = p[i];
-    } else if constexpr (sizeof(T) == 3) {
-        // one unaligned dword, [p, p + 4) for an aligned p and [p - 1, p + 3) otherwise: its one byte that is not the
-        // pixel's lies in an aligned dword that also holds a byte of the pixel, so the load cannot fault and needs no
-        // branch (the loads of several rows are in flight together).  `row` is the same for the whole wave: it stays
-        // in scalar registers and the lane adds a 32-bit offset, from row - 1 so that the offset is never negative.
-        const unsigned aligned = ((static_cast<unsigned>(reinterpret_cast<size_t>(row)) + static_cast<unsigned>(off)) & 3u) == 0u ? 1u : 0u;
-        const unsigned int w = load_dword_from_row(row, static_cast<unsigned>(off) + aligned);
-        s.w[0] = aligned != 0u ? w : w >> 8u;
     } else {
         const unsigned mis = (static_cast<unsigned>(reinterpret_cast<size_t>(row)) + static_cast<unsigned>(off)) & 3u;
         const int first = off - static_cast<int>(mis); // aligned dword that holds the pixel's first byte
@@ -1228,14 +1274,14 @@ struct ResizeJob {
             if constexpr (PACKABLE && RAW_SOURCE) {
                 // (launches of 64 x 16 tiles keep the fill of one pixel per thread: the 50-crop batch took 13.35 us this way
                 // against 13.05 us, the 16:9 crops in 64 x 32 tiles 22.9 against 23.5 us)
-                if (need != 0u && wave_rows >= 8u && packable && Access::quads_aligned(plane[i].view.src)) {
+                if (need != 0u && wave_rows >= 8u && packable) {
                     const unsigned filled = quad_filled_tile_dwords(plane[i].view.fx, plane[i].view.fy, tile_h());
                     if (filled != 0u) flags |= FLAG_QUAD_FILL;
                     tile_dwords = filled > tile_dwords ? filled : tile_dwords;
                 }
             }
             if constexpr (PACKABLE) {
-                if (need == 0u && packable && Access::quads_aligned(plane[i].view.src)) {
+                if (need == 0u && packable && (RAW_SOURCE || Access::quads_aligned(plane[i].view.src))) {
                     const unsigned packed = packed_tile_dwords(plane[i].view.fx, plane[i].view.fy, tile_h(), packed_capacity);
                     if (packed != 0u) flags |= FLAG_PACKED_TILE;
                     tile_dwords = packed > tile_dwords ? packed : tile_dwords;
@@ -1363,6 +1409,11 @@ struct ResizeJob {
             const int x2 = x1 + 1 < s.w - 1 ? x1 + 1 : s.w - 1;
             const int y2 = y1 + 1 < s.h - 1 ? y1 + 1 : s.h - 1;
             if constexpr (RAW_SOURCE && sizeof(Src) == 3) {
+                const auto pixel = [](const unsigned int w) {
+                    dev::PixelSlot<Src> px;
+                    px.w[0] = w;
+                    return to_tap(dev::slot_to_pixel<Src>(px));
+                };
                 if ((s.pitch & 3u) == 0u) {
                     // Three-byte pixels, rows a whole number of dwords apart: a column has the same alignment in every
                     // row, so the offset of the dword that holds the pixel (from one byte before the row, see
@@ -1373,11 +1424,6 @@ struct ResizeJob {
                     const bool al1 = ((base + off1) & 3u) == 0u, al2 = ((base + off2) & 3u) == 0u;
                     const unsigned voff1 = off1 + (al1 ? 1u : 0u), voff2 = off2 + (al2 ? 1u : 0u);
                     const unsigned sh1 = al1 ? 0u : 8u, sh2 = al2 ? 0u : 8u;
-                    const auto pixel = [](const unsigned int w) {
-                        dev::PixelSlot<Src> px;
-                        px.w[0] = w;
-                        return to_tap(dev::slot_to_pixel<Src>(px));
-                    };
                     for (int g = 0; g < wave_rows; g += RESIZE_GROUP_ROWS) {
                         unsigned int a[RESIZE_GROUP_ROWS], b[RESIZE_GROUP_ROWS], c[RESIZE_GROUP_ROWS], d[RESIZE_GROUP_ROWS];
 #pragma unroll
@@ -1395,8 +1441,31 @@ struct ResizeJob {
                             emit(g, k, pixel(a[K] >> sh1), pixel(b[K] >> sh2), pixel(c[K] >> sh1), pixel(d[K] >> sh2));
                         });
                     }
-                    return;
+                } else {
+                    // the same with rows at any byte: the offset and the shift of each tap (one dword instead of three bytes)
+                    const unsigned off1 = static_cast<unsigned>(x1) * 3u, off2 = static_cast<unsigned>(x2) * 3u;
+                    for (int g = 0; g < wave_rows; g += RESIZE_GROUP_ROWS) {
+                        unsigned int a[RESIZE_GROUP_ROWS], b[RESIZE_GROUP_ROWS], c[RESIZE_GROUP_ROWS], d[RESIZE_GROUP_ROWS];
+                        const char *r0[RESIZE_GROUP_ROWS], *r1[RESIZE_GROUP_ROWS];
+                        const auto starts_dword = [](const char* row, const unsigned off) { return ((static_cast<unsigned>(reinterpret_cast<size_t>(row)) + off) & 3u) == 0u; };
+                        const auto dword = [&](const char* row, const unsigned off) { return dev::load_dword_from_row(row, off + (starts_dword(row, off) ? 1u : 0u)); };
+                        const auto shifted = [&](const unsigned int w, const char* row, const unsigned off) { return starts_dword(row, off) ? w : w >> 8u; };
+#pragma unroll
+                        for (int k = 0; k < RESIZE_GROUP_ROWS; ++k) {
+                            r0[k] = window + static_cast<size_t>(__builtin_amdgcn_readlane(y1, g + k)) * s.pitch;
+                            r1[k] = window + static_cast<size_t>(__builtin_amdgcn_readlane(y2, g + k)) * s.pitch;
+                            a[k] = dword(r0[k], off1);
+                            b[k] = dword(r0[k], off2);
+                            c[k] = dword(r1[k], off1);
+                            d[k] = dword(r1[k], off2);
+                        }
+                        each_of_group([&](const auto k) {
+                            constexpr int K = decltype(k)::value;
+                            emit(g, k, pixel(shifted(a[K], r0[K], off1)), pixel(shifted(b[K], r0[K], off2)), pixel(shifted(c[K], r1[K], off1)), pixel(shifted(d[K], r1[K], off2)));
+                        });
+                    }
                 }
+                return;
             }
             for (int g = 0; g < wave_rows; g += RESIZE_GROUP_ROWS) {
                 Src a[RESIZE_GROUP_ROWS], b[RESIZE_GROUP_ROWS], c[RESIZE_GROUP_ROWS], d[RESIZE_GROUP_ROWS];
@@ -1503,17 +1572,15 @@ struct ResizeJob {
                      rows * cols <= 3 * tile_px + 256;
             tile_x0 = sx_lo;
             if constexpr (PACKABLE) {
-                // A box that is not worth a tile of float taps as above (down-scaling: few taps per source pixel), of an image
-                // that starts at a whole dword with rows a whole number of dwords apart: the aligned groups of four pixels
-                // that cover the box's columns, in the rows of it that exist, each fetched by one thread with one load (two
+                // A box that is not worth a tile of float taps as above (down-scaling: few taps per source pixel): the groups of
+                // four pixels that cover the box's columns, in the rows of it that exist, each fetched by one thread with one load (two
                 // for 4:2:0 sources) through a descriptor of the whole parent image (a group that reaches past the image's
                 // last row end reads zeros there and cannot fault).  Pixels as they lie in memory are kept as one dword
                 // each; pixels that are computed (operations fused before the resize) are kept as float taps, computed once
                 // per source pixel.  Thread t takes groups t, t + 256, ... of the box (rows of `quads` groups); the loads of up
                 // to four of them are issued before the first is used, so a box costs one memory round trip.
                 const int box_px = rows * cols;
-                if (!staged && (job_flags & FLAG_PACKED_TILE) != 0u && box_px <= PACKED_MAX_RATIO * tile_px + 256 &&
-                    ((static_cast<unsigned>(reinterpret_cast<size_t>(s.data)) | s.pitch) & 3u) == 0u) {
+                if (!staged && (job_flags & FLAG_PACKED_TILE) != 0u && box_px <= PACKED_MAX_RATIO * tile_px + 256 && (RAW_SOURCE || Access::quads_aligned(s))) {
                     const int last_c = sx_lo + cols - 1 < s.w - 1 ? sx_lo + cols - 1 : s.w - 1; // window columns sx_lo .. last_c
                     const int last_r = sy_lo + rows - 1 < s.h - 1 ? sy_lo + rows - 1 : s.h - 1;
                     const int q_lo = (s.ox + sx_lo) >> 2;
@@ -1533,46 +1600,51 @@ struct ResizeJob {
                         const unsigned m = static_cast<unsigned>(1048576.0f * __builtin_amdgcn_rcpf(static_cast<float>(quads))) + 2u;
                         const __amdgpu_buffer_rsrc_t image = Access::quad_buffer(s);
                         const int py0 = s.oy + sy_lo;
-                        for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform)
-                            typename Access::Quad raw[PASSES];
-                            // (no branch between the loads: groups past the box's last repeat it, from the cache)
-#pragma unroll
-                            for (int u = 0; u < PASSES; ++u) {
-                                const int wanted = first + BLOCK_THREADS * u + tid;
-                                const int item = wanted < items ? wanted : items - 1;
-                                const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
-                                raw[u] = Access::load_quad(image, s, q_lo + (item - r * quads), py0 + r);
-                            }
-#pragma unroll
-                            for (int u = 0; u < PASSES; ++u) {
-                                if (first + BLOCK_THREADS * u + 64 * wave_of_block < items) { // (uniform: some group of this wave's pass exists)
+                        const auto fill = [&](const auto any) {
+                            constexpr bool ANY = decltype(any)::value;
+                            for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform)
+                                typename Access::template RawQuad<ANY> raw[PASSES];
+                                // (no branch between the loads: groups past the box's last repeat it, from the cache)
+    #pragma unroll
+                                for (int u = 0; u < PASSES; ++u) {
                                     const int wanted = first + BLOCK_THREADS * u + tid;
                                     const int item = wanted < items ? wanted : items - 1;
-                                    if constexpr (RAW_SOURCE) {
-                                        unsigned int px[4];
-                                        Access::quad_dwords(raw[u], px);
-                                        dev::u32x4 piece;
-                                        piece.x = px[0]; piece.y = px[1]; piece.z = px[2]; piece.w = px[3];
-                                        *reinterpret_cast<dev::u32x4*>(tile + item * 4) = piece;
-                                    } else {
-                                        typename SrcView::Pixel px[4];
-                                        Access::quad_pixels(raw[u], px);
-                                        unsigned int taps[4 * SLOT];
-#pragma unroll
-                                        for (int k = 0; k < 4; ++k) {
-                                            const Tap t = to_tap(dev::apply_tail(v.pre, px[k]));
-                                            __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
-                                        }
-#pragma unroll
-                                        for (int k = 0; k < SLOT; ++k) {
+                                    const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
+                                    Access::template load_quad<ANY>(image, s, q_lo + (item - r * quads), py0 + r, raw[u]);
+                                }
+    #pragma unroll
+                                for (int u = 0; u < PASSES; ++u) {
+                                    if (first + BLOCK_THREADS * u + 64 * wave_of_block < items) { // (uniform: some group of this wave's pass exists)
+                                        const int wanted = first + BLOCK_THREADS * u + tid;
+                                        const int item = wanted < items ? wanted : items - 1;
+                                        if constexpr (RAW_SOURCE) {
+                                            unsigned int px[4];
+                                            Access::template quad_dwords<ANY>(raw[u], px);
                                             dev::u32x4 piece;
-                                            piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
-                                            reinterpret_cast<dev::u32x4*>(tile + item * 4 * SLOT)[k] = piece;
+                                            piece.x = px[0]; piece.y = px[1]; piece.z = px[2]; piece.w = px[3];
+                                            *reinterpret_cast<dev::u32x4*>(tile + item * 4) = piece;
+                                        } else {
+                                            typename SrcView::Pixel px[4];
+                                            Access::template quad_pixels<ANY>(raw[u], px);
+                                            unsigned int taps[4 * SLOT];
+    #pragma unroll
+                                            for (int k = 0; k < 4; ++k) {
+                                                const Tap t = to_tap(dev::apply_tail(v.pre, px[k]));
+                                                __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
+                                            }
+    #pragma unroll
+                                            for (int k = 0; k < SLOT; ++k) {
+                                                dev::u32x4 piece;
+                                                piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
+                                                reinterpret_cast<dev::u32x4*>(tile + item * 4 * SLOT)[k] = piece;
+                                            }
                                         }
                                     }
                                 }
                             }
-                        }
+                        };
+                        if (Access::quads_aligned(s)) fill(std::false_type{});
+                        else if constexpr (RAW_SOURCE) fill(std::true_type{});
                     }
                 }
             }
@@ -1595,17 +1667,14 @@ struct ResizeJob {
                 const int pass_rows = 64 >> lane_cols_log2;            // rows of a wave's pass
                 const int lane_row = wave * pass_rows + (lane >> lane_cols_log2); // this lane's row in the block's first pass
                 const int block_rows = WAVES * pass_rows;              // rows of a block's pass
-                bool rows_alike = false;
-                if constexpr (RAW_SOURCE && sizeof(Src) == 3) rows_alike = (s.pitch & 3u) == 0u;
                 bool staged_by_item = false;
                 if constexpr (RAW_SOURCE && PACKABLE) {
-                    // Three-byte pixels of an image that starts at a whole dword, rows a whole number of dwords apart: the tile
-                    // is filled from the aligned groups of four pixels (twelve bytes, one load) that cover the box's columns,
-                    // read through a descriptor of the whole parent image, so a thread converts four pixels per load and
-                    // address instead of one.  The tile's column 0 is the first group's first pixel, a row holds the groups and
+                    // Three-byte pixels: the tile is filled from the groups of four pixels (twelve bytes, one load) that cover the
+                    // box's columns, read through a descriptor of the whole parent image, so a thread converts four pixels per
+                    // load and address instead of one.  The tile's column 0 is the first group's first pixel, a row holds the groups and
                     // room for one more; rows past the window's last are the last one again, and where the box reaches past
                     // the window's last column, the thread that fetched that column writes its copy behind it.
-                    if ((job_flags & FLAG_QUAD_FILL) != 0u && ((static_cast<unsigned>(reinterpret_cast<size_t>(s.data)) | s.pitch) & 3u) == 0u) {
+                    if ((job_flags & FLAG_QUAD_FILL) != 0u) {
                         const int last_c = sx_lo + cols - 1 < s.w - 1 ? sx_lo + cols - 1 : s.w - 1;
                         const int q_lo = (s.ox + sx_lo) >> 2;
                         const int quads = ((s.ox + last_c) >> 2) - q_lo + 1;
@@ -1624,61 +1693,65 @@ struct ResizeJob {
                             // the window's last column inside its group, and where its copies go from the start of that group
                             const int edge_pixel = (s.ox + s.w - 1) & 3;
                             const int edge_slot = (s.w - tile_x0 - 4 * (quads - 1)) * SLOT;
-                            constexpr int PASSES = 1;
-                            for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform: one turn)
-                                typename Access::Quad raw[PASSES];
-                                int at[PASSES];
-                                bool last_group[PASSES];
-#pragma unroll
-                                for (int u = 0; u < PASSES; ++u) {
-                                    const int wanted = first + BLOCK_THREADS * u + tid;
-                                    const int item = wanted < items ? wanted : items - 1;
-                                    const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
-                                    const int q = item - r * quads;
-                                    const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
-                                    raw[u] = Access::load_quad(image, s, q_lo + q, s.oy + sy);
-                                    at[u] = (r * row_px + 4 * q) * SLOT;
-                                    last_group[u] = q == quads - 1;
-                                }
-#pragma unroll
-                                for (int u = 0; u < PASSES; ++u) {
-                                    if (first + BLOCK_THREADS * u + 64 * wave < items) { // (uniform: some group of this wave's pass exists)
-                                        Src px[4];
-                                        Access::quad_pixels(raw[u], px);
-                                        unsigned int taps[4 * SLOT];
-#pragma unroll
-                                        for (int k = 0; k < 4; ++k) {
-                                            const Tap t = to_tap(px[k]);
-                                            __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
-                                        }
-#pragma unroll
-                                        for (int k = 0; k < SLOT; ++k) {
-                                            dev::u32x4 piece;
-                                            piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
-                                            reinterpret_cast<dev::u32x4*>(tile + at[u])[k] = piece;
-                                        }
-                                        // The copies of the window's last column behind it, by the thread that holds that column (its
-                                        // row's last group), after its own stores: the copy lies inside that group or in the room
-                                        // behind it, which no other thread writes.
-                                        if (behind > 0) { // (uniform)
-                                            Src edge = px[0];
-                                            if (edge_pixel == 1) edge = px[1];
-                                            if (edge_pixel == 2) edge = px[2];
-                                            if (edge_pixel == 3) edge = px[3];
-                                            if (last_group[u]) {
-                                                for (int j = 0; j < behind; ++j) store_tap(tile + at[u] + edge_slot + j * SLOT, to_tap(edge));
+                            const auto fill = [&](const auto any) {
+                                constexpr bool ANY = decltype(any)::value;
+                                constexpr int PASSES = 1;
+                                for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform: one turn)
+                                    typename Access::template RawQuad<ANY> raw[PASSES];
+                                    int at[PASSES];
+                                    bool last_group[PASSES];
+    #pragma unroll
+                                    for (int u = 0; u < PASSES; ++u) {
+                                        const int wanted = first + BLOCK_THREADS * u + tid;
+                                        const int item = wanted < items ? wanted : items - 1;
+                                        const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
+                                        const int q = item - r * quads;
+                                        const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
+                                        Access::template load_quad<ANY>(image, s, q_lo + q, s.oy + sy, raw[u]);
+                                        at[u] = (r * row_px + 4 * q) * SLOT;
+                                        last_group[u] = q == quads - 1;
+                                    }
+    #pragma unroll
+                                    for (int u = 0; u < PASSES; ++u) {
+                                        if (first + BLOCK_THREADS * u + 64 * wave < items) { // (uniform: some group of this wave's pass exists)
+                                            Src px[4];
+                                            Access::template quad_pixels<ANY>(raw[u], px);
+                                            unsigned int taps[4 * SLOT];
+    #pragma unroll
+                                            for (int k = 0; k < 4; ++k) {
+                                                const Tap t = to_tap(px[k]);
+                                                __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
+                                            }
+    #pragma unroll
+                                            for (int k = 0; k < SLOT; ++k) {
+                                                dev::u32x4 piece;
+                                                piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
+                                                reinterpret_cast<dev::u32x4*>(tile + at[u])[k] = piece;
+                                            }
+                                            // The copies of the window's last column behind it, by the thread that holds that column (its
+                                            // row's last group), after its own stores: the copy lies inside that group or in the room
+                                            // behind it, which no other thread writes.
+                                            if (behind > 0) { // (uniform)
+                                                Src edge = px[0];
+                                                if (edge_pixel == 1) edge = px[1];
+                                                if (edge_pixel == 2) edge = px[2];
+                                                if (edge_pixel == 3) edge = px[3];
+                                                if (last_group[u]) {
+                                                    for (int j = 0; j < behind; ++j) store_tap(tile + at[u] + edge_slot + j * SLOT, to_tap(edge));
+                                                }
                                             }
                                         }
                                     }
                                 }
-                            }
+                            };
+                            if (Access::quads_aligned(s)) fill(std::false_type{});
+                            else fill(std::true_type{});
                         }
                     }
                 }
                 if constexpr (RAW_SOURCE && sizeof(Src) == 3) {
-                    if (rows_alike && !staged_by_item) {
-                        // Three-byte pixels, rows a whole number of dwords apart (the common case): the box's pixels in row-major
-                        // order, thread t takes pixels t, t + 256, ..., the loads of all of them in flight before the first
+                    if (!staged_by_item) {
+                        // Three-byte pixels, rows at any byte: the box's pixels in row-major order, thread t takes pixels t, t + 256, ..., the loads of all of them in flight before the first
                         // is stored, so a box costs one memory round trip with every lane busy (with the lanes
                         // laid over columns, a box of 35 columns leaves 29 lanes of every wave idle and takes five passes of four
                         // rows).  item / cols comes from a multiplication by the reciprocal instruction's result: (item + 0.5) / cols
@@ -1704,9 +1777,9 @@ struct ResizeJob {
                                     const int c = item - r * cols;
                                     const int sx = sx_lo + c < s.w - 1 ? sx_lo + c : s.w - 1;
                                     const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
-                                    const unsigned off = static_cast<unsigned>(sx) * 3u;
+                                    const unsigned off = static_cast<unsigned>(sy) * s.pitch + static_cast<unsigned>(sx) * 3u;
                                     const bool aligned = ((base + off) & 3u) == 0u;
-                                    got[u] = dev::load_dword_from_row(window, static_cast<unsigned>(sy) * s.pitch + off + (aligned ? 1u : 0u));
+                                    got[u] = dev::load_dword_from_row(window, off + (aligned ? 1u : 0u));
                                     shift[u] = aligned ? 0u : 8u;
                                     at[u] = (r * stride + c) * SLOT;
                                 }
@@ -1725,51 +1798,38 @@ struct ResizeJob {
                         else stage_passes(std::integral_constant<int, 8>{});
                     }
                 }
-                for (int c = lane & (lane_cols - 1); c < cols && !staged_by_item; c += lane_cols) {
-                    const int sx = sx_lo + c < s.w - 1 ? sx_lo + c : s.w - 1;
-                    // three-byte pixels, rows a whole number of dwords apart: a column has the same alignment in every
-                    // row, so a lane's offset and the shift that takes the pixel out of its dword are found once per column
-                    const unsigned off = static_cast<unsigned>(sx) * static_cast<unsigned>(sizeof(Src));
-                    const bool aligned = ((static_cast<unsigned>(reinterpret_cast<size_t>(window)) + off) & 3u) == 0u;
-                    const unsigned voff = off + (aligned ? 1u : 0u); // from one byte before the row
-                    for (int first = 0; first < rows; first += block_rows * STAGE_ROWS) { // (uniform)
-                        if constexpr (RAW_SOURCE) {
-                            dev::PixelSlot<Src> px[STAGE_ROWS];
-#pragma unroll
-                            for (int u = 0; u < STAGE_ROWS; ++u) {
-                                const int wanted = first + block_rows * u + lane_row;
-                                const int r = wanted < rows ? wanted : rows - 1;
-                                const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
-                                if constexpr (sizeof(Src) == 3) {
-                                    // (the row's offset from the window's first pixel fits the lane's 32 bits: the host stages
-                                    // tiles of three-byte pixels only for windows that span less than 4 GiB, FLAG_OFFSETS_32)
-                                    if (rows_alike) {
-                                        const unsigned int w = dev::load_dword_from_row(window, static_cast<unsigned>(sy) * s.pitch + voff);
-                                        px[u].w[0] = aligned ? w : w >> 8u;
-                                    } else {
-                                        px[u] = dev::load_pixel_slot<Src>(window, static_cast<int>(static_cast<unsigned>(sy) * s.pitch + off), valid_lo, valid_hi);
-                                    }
-                                } else {
-                                    px[u] = dev::load_pixel_slot<Src>(window + static_cast<size_t>(sy) * s.pitch, static_cast<int>(off), valid_lo, valid_hi);
+                if constexpr (!(RAW_SOURCE && sizeof(Src) == 3)) { // (three-byte pixels have been staged above)
+                    for (int c = lane & (lane_cols - 1); c < cols; c += lane_cols) {
+                        const int sx = sx_lo + c < s.w - 1 ? sx_lo + c : s.w - 1;
+                        const int off = sx * static_cast<int>(sizeof(Src));
+                        for (int first = 0; first < rows; first += block_rows * STAGE_ROWS) { // (uniform)
+                            if constexpr (RAW_SOURCE) {
+                                dev::PixelSlot<Src> px[STAGE_ROWS];
+    #pragma unroll
+                                for (int u = 0; u < STAGE_ROWS; ++u) {
+                                    const int wanted = first + block_rows * u + lane_row;
+                                    const int r = wanted < rows ? wanted : rows - 1;
+                                    const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
+                                    px[u] = dev::load_pixel_slot<Src>(window + static_cast<size_t>(sy) * s.pitch, off, valid_lo, valid_hi);
                                 }
-                            }
-#pragma unroll
-                            for (int u = 0; u < STAGE_ROWS; ++u) {
-                                const int wanted = first + block_rows * u + lane_row;
-                                const int r = wanted < rows ? wanted : rows - 1;
-                                store_tap(tile + (r * stride + c) * SLOT, to_tap(dev::slot_to_pixel<Src>(px[u])));
-                            }
-                        } else {
-                            Src px[STAGE_ROWS];
-#pragma unroll
-                            for (int u = 0; u < STAGE_ROWS; ++u) {
-                                const int r = first + block_rows * u + lane_row;
-                                if (r < rows) px[u] = fetch(v, sx, sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1);
-                            }
-#pragma unroll
-                            for (int u = 0; u < STAGE_ROWS; ++u) {
-                                const int r = first + block_rows * u + lane_row;
-                                if (r < rows) store_tap(tile + (r * stride + c) * SLOT, to_tap(px[u]));
+    #pragma unroll
+                                for (int u = 0; u < STAGE_ROWS; ++u) {
+                                    const int wanted = first + block_rows * u + lane_row;
+                                    const int r = wanted < rows ? wanted : rows - 1;
+                                    store_tap(tile + (r * stride + c) * SLOT, to_tap(dev::slot_to_pixel<Src>(px[u])));
+                                }
+                            } else {
+                                Src px[STAGE_ROWS];
+    #pragma unroll
+                                for (int u = 0; u < STAGE_ROWS; ++u) {
+                                    const int r = first + block_rows * u + lane_row;
+                                    if (r < rows) px[u] = fetch(v, sx, sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1);
+                                }
+    #pragma unroll
+                                for (int u = 0; u < STAGE_ROWS; ++u) {
+                                    const int r = first + block_rows * u + lane_row;
+                                    if (r < rows) store_tap(tile + (r * stride + c) * SLOT, to_tap(px[u]));
+                                }
                             }
                         }
                     }

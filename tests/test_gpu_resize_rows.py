@@ -1,0 +1,40 @@
+"""Resizes of three-byte pixels whose rows start at any byte of a dword, by each way the resize kernel takes its taps: tiles of
+float taps filled pixel by pixel (64 x 16) and in groups of four (64 x 32 and taller), tiles of packed pixels (down-scaling),
+taps straight from memory (strong down-scaling); regions that touch the image's first and last bytes, where a group of four
+pixels is cut by the image's end.  The image lies at the end of its allocation's used part, with a pattern around it; against the
+CPU oracle, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import same_bits
+
+pytestmark = pytest.mark.gpu
+ONE, ZERO = (1.0,) * 3, (0.0,) * 3
+
+
+def at_byte(img, start, extra):
+    """`img` (h, w, 3) in device memory, its first pixel `start` bytes behind a dword, rows `extra` bytes further apart than tight."""
+    h, w, _ = img.shape
+    pitch = 3 * w + extra
+    flat = np.full(start + h * pitch, 170, np.uint8)
+    rows = flat[start:].reshape(h, pitch)
+    rows[:, :3 * w] = img.reshape(h, 3 * w)
+    t = torch.from_numpy(flat).cuda()
+    return torch.as_strided(t, (h, w, 3), (pitch, 3, 1), start)
+
+
+@pytest.mark.parametrize("w,start,extra", [(301, 0, 0), (302, 1, 0), (303, 2, 0), (300, 3, 0), (300, 0, 1), (299, 3, 2), (304, 0, 0)])
+# up-scaling in small tiles; in taller tiles (many blocks); packed tiles; taps from memory, with and without lines touched first
+@pytest.mark.parametrize("dst,side,n", [((130, 75), (61, 40), 3), ((700, 900), (299, 200), 10), ((128, 90), (200, 150), 3), ((60, 60), (290, 200), 2), ((66, 33), (299, 201), 2), ((7, 5), (3, 2), 2)])
+def test_rows_at_any_byte(fk, oracle, w, start, extra, dst, side, n):
+    h = 203
+    img = oracle.bytes(900 + w + start, (h, w, 3))
+    sw, sh = min(side[0], w), side[1]
+    corners = [(0, 0), (w - sw, h - sh), (w - sw, 0), (0, h - sh), (1, 1), (w - sw - 1, h - sh - 1)]
+    rects = [(max(0, min(x, w - sw)), max(0, min(y, h - sh)), sw, sh) for x, y in (corners[i % len(corners)] for i in range(n))]
+    src = at_byte(img, start, extra)
+    for aspect in (fk.IGNORE_AR, fk.PRESERVE_AR):
+        out = torch.full((n, dst[1], dst[0], 3), -1.0, device="cuda")
+        fk.crop_resize_muls_bgr_tensor(src, rects, out, aspect, (3, 2, 1), ONE, ZERO, ONE)
+        assert same_bits(out.cpu().numpy(), oracle.crop_resize_muls_bgr_tensor(img, rects, dst, aspect, (3, 2, 1), ONE, ZERO, ONE)), aspect
