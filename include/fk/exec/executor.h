@@ -200,7 +200,7 @@ struct JobOf {
                 job.grid_y = job.plan(used, max_h, resize_wave_rows_override(), resize_packed_capacity());
                 // x-neighbouring tiles in pairs on one XCD (FK_RESIZE_NO_PAIRS switches it off: for measurements)
                 const ResizeSwitches& switches = resize_switches();
-                if (switches.no_quad_fill) job.flags &= ~FLAG_QUAD_FILL;
+                if (switches.no_quad_fill) job.flags &= ~(FLAG_QUAD_FILL | FLAG_QUAD_FILL_ANY);
                 if (job.tile_dwords != 0u && switches.lds_dwords > job.tile_dwords) job.tile_dwords = switches.lds_dwords;
                 if (!switches.no_pairs) {
                     const unsigned gx = job.grid_x;

@@ -770,7 +770,7 @@ __device__ __attribute__((always_inline)) inline void fill_default(const Out& ou
 // ---- pointwise ---------------------------------------------------------------------------------------------------
 // FLAG_GROUP_IO: a thread's K pixels move as wide accesses, at whatever byte alignment; FLAG_VECTOR_IO: at their natural
 // alignment as well
-enum : unsigned { FLAG_VECTOR_IO = 1u, FLAG_GROUP_IO = 512u, FLAG_STREAM_STORES = 2u, FLAG_SOURCE_TILE = 4u, FLAG_WHOLE_BOX = 8u, FLAG_PACKED_TILE = 16u, FLAG_OFFSETS_32 = 32u, FLAG_PAIR_COLUMNS = 64u, FLAG_PAIR_TILES = 128u, FLAG_QUAD_FILL = 256u };
+enum : unsigned { FLAG_VECTOR_IO = 1u, FLAG_GROUP_IO = 512u, FLAG_STREAM_STORES = 2u, FLAG_SOURCE_TILE = 4u, FLAG_WHOLE_BOX = 8u, FLAG_PACKED_TILE = 16u, FLAG_OFFSETS_32 = 32u, FLAG_PAIR_COLUMNS = 64u, FLAG_PAIR_TILES = 128u, FLAG_QUAD_FILL = 256u, FLAG_PACKED_TILE_ANY = 1024u, FLAG_QUAD_FILL_ANY = 2048u };
 
 constexpr int max_of(const int a) { return a; }
 template <typename... Rest>
@@ -1186,7 +1186,8 @@ struct ResizeJob {
     unsigned grid_x, grid_y;
     // FLAG_STREAM_STORES: large output whose rows start at whole dwords; FLAG_SOURCE_TILE / FLAG_PACKED_TILE: some plane's
     // tiles are staged in LDS, as float taps / as packed pixels, which decides how much LDS the launch asks for (a
-    // divergent launch shares one LDS size between all its jobs).
+    // divergent launch shares one LDS size between all its jobs); FLAG_QUAD_FILL: tiles of float taps filled from groups of four pixels.
+    // FLAG_PACKED_TILE and FLAG_QUAD_FILL are for images whose rows start at whole dwords, the flags named _ANY for those of other images.
     unsigned flags;
     // Rows of the tile that each of the block's four waves computes (4, 8 or 16: the tile is 64 x 4 * wave_rows).
     // What a wave does once (the tile's source box, its lanes' columns) is shared by more rows in a taller tile; a
@@ -1196,7 +1197,7 @@ struct ResizeJob {
     // many blocks a CU holds.  tile_dwords is the room for a source tile (a tile that needs more reads its taps directly).
     unsigned tile_dwords;
     Defaults defaults;
-    size_t lds_bytes() const { return (flags & (FLAG_SOURCE_TILE | FLAG_PACKED_TILE)) != 0u ? static_cast<size_t>(tile_dwords) * 4 + 16 : 0; }
+    size_t lds_bytes() const { return (flags & (FLAG_SOURCE_TILE | FLAG_PACKED_TILE | FLAG_PACKED_TILE_ANY)) != 0u ? static_cast<size_t>(tile_dwords) * 4 + 16 : 0; }
     int tile_h() const { return (BLOCK_THREADS / 64) * static_cast<int>(wave_rows); }
     // dwords a tile of a plane with these factors takes when staged, 0 when it is not worth staging (same rule as the
     // kernel applies per tile)
@@ -1276,14 +1277,14 @@ struct ResizeJob {
                 // against 13.05 us, the 16:9 crops in 64 x 32 tiles 22.9 against 23.5 us)
                 if (need != 0u && wave_rows >= 8u && packable) {
                     const unsigned filled = quad_filled_tile_dwords(plane[i].view.fx, plane[i].view.fy, tile_h());
-                    if (filled != 0u) flags |= FLAG_QUAD_FILL;
+                    if (filled != 0u) flags |= Access::quads_aligned(plane[i].view.src) ? FLAG_QUAD_FILL : FLAG_QUAD_FILL_ANY;
                     tile_dwords = filled > tile_dwords ? filled : tile_dwords;
                 }
             }
             if constexpr (PACKABLE) {
                 if (need == 0u && packable && (RAW_SOURCE || Access::quads_aligned(plane[i].view.src))) {
                     const unsigned packed = packed_tile_dwords(plane[i].view.fx, plane[i].view.fy, tile_h(), packed_capacity);
-                    if (packed != 0u) flags |= FLAG_PACKED_TILE;
+                    if (packed != 0u) flags |= Access::quads_aligned(plane[i].view.src) ? FLAG_PACKED_TILE : FLAG_PACKED_TILE_ANY;
                     tile_dwords = packed > tile_dwords ? packed : tile_dwords;
                 }
             }
@@ -1580,7 +1581,7 @@ struct ResizeJob {
                 // per source pixel.  Thread t takes groups t, t + 256, ... of the box (rows of `quads` groups); the loads of up
                 // to four of them are issued before the first is used, so a box costs one memory round trip.
                 const int box_px = rows * cols;
-                if (!staged && (job_flags & FLAG_PACKED_TILE) != 0u && box_px <= PACKED_MAX_RATIO * tile_px + 256 && (RAW_SOURCE || Access::quads_aligned(s))) {
+                if (!staged && (job_flags & (Access::quads_aligned(s) ? FLAG_PACKED_TILE : FLAG_PACKED_TILE_ANY)) != 0u && box_px <= PACKED_MAX_RATIO * tile_px + 256) {
                     const int last_c = sx_lo + cols - 1 < s.w - 1 ? sx_lo + cols - 1 : s.w - 1; // window columns sx_lo .. last_c
                     const int last_r = sy_lo + rows - 1 < s.h - 1 ? sy_lo + rows - 1 : s.h - 1;
                     const int q_lo = (s.ox + sx_lo) >> 2;
@@ -1605,14 +1606,14 @@ struct ResizeJob {
                             for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform)
                                 typename Access::template RawQuad<ANY> raw[PASSES];
                                 // (no branch between the loads: groups past the box's last repeat it, from the cache)
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < PASSES; ++u) {
                                     const int wanted = first + BLOCK_THREADS * u + tid;
                                     const int item = wanted < items ? wanted : items - 1;
                                     const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
                                     Access::template load_quad<ANY>(image, s, q_lo + (item - r * quads), py0 + r, raw[u]);
                                 }
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < PASSES; ++u) {
                                     if (first + BLOCK_THREADS * u + 64 * wave_of_block < items) { // (uniform: some group of this wave's pass exists)
                                         const int wanted = first + BLOCK_THREADS * u + tid;
@@ -1627,12 +1628,12 @@ struct ResizeJob {
                                             typename SrcView::Pixel px[4];
                                             Access::template quad_pixels<ANY>(raw[u], px);
                                             unsigned int taps[4 * SLOT];
-    #pragma unroll
+#pragma unroll
                                             for (int k = 0; k < 4; ++k) {
                                                 const Tap t = to_tap(dev::apply_tail(v.pre, px[k]));
                                                 __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
                                             }
-    #pragma unroll
+#pragma unroll
                                             for (int k = 0; k < SLOT; ++k) {
                                                 dev::u32x4 piece;
                                                 piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
@@ -1674,7 +1675,7 @@ struct ResizeJob {
                     // load and address instead of one.  The tile's column 0 is the first group's first pixel, a row holds the groups and
                     // room for one more; rows past the window's last are the last one again, and where the box reaches past
                     // the window's last column, the thread that fetched that column writes its copy behind it.
-                    if ((job_flags & FLAG_QUAD_FILL) != 0u) {
+                    if ((job_flags & (Access::quads_aligned(s) ? FLAG_QUAD_FILL : FLAG_QUAD_FILL_ANY)) != 0u) {
                         const int last_c = sx_lo + cols - 1 < s.w - 1 ? sx_lo + cols - 1 : s.w - 1;
                         const int q_lo = (s.ox + sx_lo) >> 2;
                         const int quads = ((s.ox + last_c) >> 2) - q_lo + 1;
@@ -1700,7 +1701,7 @@ struct ResizeJob {
                                     typename Access::template RawQuad<ANY> raw[PASSES];
                                     int at[PASSES];
                                     bool last_group[PASSES];
-    #pragma unroll
+#pragma unroll
                                     for (int u = 0; u < PASSES; ++u) {
                                         const int wanted = first + BLOCK_THREADS * u + tid;
                                         const int item = wanted < items ? wanted : items - 1;
@@ -1711,18 +1712,18 @@ struct ResizeJob {
                                         at[u] = (r * row_px + 4 * q) * SLOT;
                                         last_group[u] = q == quads - 1;
                                     }
-    #pragma unroll
+#pragma unroll
                                     for (int u = 0; u < PASSES; ++u) {
                                         if (first + BLOCK_THREADS * u + 64 * wave < items) { // (uniform: some group of this wave's pass exists)
                                             Src px[4];
                                             Access::template quad_pixels<ANY>(raw[u], px);
                                             unsigned int taps[4 * SLOT];
-    #pragma unroll
+#pragma unroll
                                             for (int k = 0; k < 4; ++k) {
                                                 const Tap t = to_tap(px[k]);
                                                 __builtin_memcpy(taps + k * SLOT, &t, sizeof(Tap));
                                             }
-    #pragma unroll
+#pragma unroll
                                             for (int k = 0; k < SLOT; ++k) {
                                                 dev::u32x4 piece;
                                                 piece.x = taps[4 * k]; piece.y = taps[4 * k + 1]; piece.z = taps[4 * k + 2]; piece.w = taps[4 * k + 3];
@@ -1805,14 +1806,14 @@ struct ResizeJob {
                         for (int first = 0; first < rows; first += block_rows * STAGE_ROWS) { // (uniform)
                             if constexpr (RAW_SOURCE) {
                                 dev::PixelSlot<Src> px[STAGE_ROWS];
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < STAGE_ROWS; ++u) {
                                     const int wanted = first + block_rows * u + lane_row;
                                     const int r = wanted < rows ? wanted : rows - 1;
                                     const int sy = sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1;
                                     px[u] = dev::load_pixel_slot<Src>(window + static_cast<size_t>(sy) * s.pitch, off, valid_lo, valid_hi);
                                 }
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < STAGE_ROWS; ++u) {
                                     const int wanted = first + block_rows * u + lane_row;
                                     const int r = wanted < rows ? wanted : rows - 1;
@@ -1820,12 +1821,12 @@ struct ResizeJob {
                                 }
                             } else {
                                 Src px[STAGE_ROWS];
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < STAGE_ROWS; ++u) {
                                     const int r = first + block_rows * u + lane_row;
                                     if (r < rows) px[u] = fetch(v, sx, sy_lo + r < s.h - 1 ? sy_lo + r : s.h - 1);
                                 }
-    #pragma unroll
+#pragma unroll
                                 for (int u = 0; u < STAGE_ROWS; ++u) {
                                     const int r = first + block_rows * u + lane_row;
                                     if (r < rows) store_tap(tile + (r * stride + c) * SLOT, to_tap(px[u]));
