@@ -302,6 +302,8 @@ struct JobOf {
                 job.out_z_stride = out.z_stride;
             }
             job.packs_rows = 0u;
+            job.tile_dwords = job.plan_tiles();
+            if (job.tile_dwords != 0u) job.xcd_bands = 1u;
             if constexpr (decltype(job)::PACKS_ROWS) {
                 const auto out = OutOf<Receiver>::make(receiver);
                 job.packs_rows = (aligned_to(out.data, 4) && out.pitch % 4u == 0u && out.z_stride % 4u == 0u) ? 1u : 0u;

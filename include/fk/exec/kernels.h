@@ -20,6 +20,7 @@
 #define FK_EXEC_KERNELS_H
 
 #include "fk/exec/views.h"
+#include "fk/ops/warping.h"
 
 // clang emits a host-side stub for every __global__ function that refers to this runtime entry point; kernels are
 // launched through fkrt_launch (which calls it with the stub's address), so only the declaration is needed here.  A
@@ -1969,6 +1970,38 @@ __device__ __attribute__((always_inline)) inline void xcd_band_block(unsigned& b
 }
 } // namespace dev
 
+// Warps of images of three-byte pixels take their taps from LDS where the output is large and slanted: a block owns a tile of 64 x 16
+// outputs, a lane one column of it in each of its wave's four rows.  The source box of the tile comes from its four corners (the
+// matrix maps lines to lines, so every tap lies between them), its pixels are fetched in groups of four and kept as they are, one
+// dword each: a pixel's four taps are two reads of neighbouring dwords.  What bounded the gathers: four of them per pixel keep the
+// address units busy, the longer the more lines a slanted row of 64 crosses, and each computes a 64-bit address.  Tiles of float taps,
+// converted once per source pixel, had been slower than the gathers; pixels as they are cost the fill next to nothing.  Eight rows per
+// wave are slower: fewer blocks, larger boxes (3840x2160 by 5 degrees 25.1 us against 24.1, 4.9 TB/s of 124 MB against 5.2).
+template <typename Sender>
+struct WarpOfPixels : std::false_type {};
+template <WarpType WT, typename T>
+struct WarpOfPixels<ReadBack<Warping<WT, Read<PerThreadRead<ND::_2D, T>>>>> : std::bool_constant<sizeof(T) == 3 && cn<T> == 3> {
+    static constexpr WarpType TYPE = WT;
+    using Coords = WarpingCoords<WT>;
+    using Params = WarpingParameters<WT>;
+    using Pixel = T;
+    static PlainView<T> view(const RawPtr<ND::_2D, T>& p) {
+        const int w = static_cast<int>(p.dims.width), h = static_cast<int>(p.dims.height);
+        return PlainView<T>{ p.data, p.dims.pitch, w, h, 0, 0, w, h };
+    }
+};
+constexpr int WARP_TILE_W = 64, WARP_ROWS = 4, WARP_TILE_H = 4 * WARP_ROWS; // (rows of a wave, of a block)
+// Where the lines of a launch's rule lie (MI355X, four gathers per pixel against tiles, us):
+//  - boxes of up to 8192 pixels (32 KiB): 3840x2160 to 2560x1440 by 20 degrees, boxes of 5900, 21.3 -> 15.2; to 1920x1080 by 10 degrees,
+//    boxes of 7300, 12.9 -> 10.8; larger ones leave fewer than five blocks per CU;
+//  - 1024 tiles and more: 1920x1080 (2040 tiles) by 5 degrees 8.6 -> 7.9, 1228x1000 (1260) 8.6 -> 8.3; 1280x720 (900) 4.8 -> 5.3;
+//  - rows of a tile that cross four source rows and more (their gathers touch as many lines), eight for a perspective map (its
+//    division per pixel, and per corner, keeps the vector units busy in both forms): 3840x2160 by 0, 5 and 20 degrees 24.9 -> 25.6, 27.1 -> 24.1
+//    and 45.1 -> 25.1, with a tilt 28.5 -> 29.7, 27.1 -> 28.0 and 45.1 -> 28.2.
+constexpr unsigned WARP_TILE_DWORDS = 8192, WARP_MIN_BLOCKS = 1024;
+constexpr float WARP_SLANT_AFFINE = 4.f, WARP_SLANT_PERSPECTIVE = 8.f;
+constexpr float WARP_BOX_MARGIN = 0.0625f;   // the corners' and the taps' coordinates are rounded; what lies outside is taken from memory
+
 constexpr unsigned GENERIC_WIDE_MIN_ELEMS = 1u << 22;
 template <typename Sender, typename Receiver>
 struct GenericJob {
@@ -2004,7 +2037,47 @@ struct GenericJob {
     char* out_data;      // element (0, 0, 0) of the receiver, bytes between its rows and between its planes
     unsigned out_pitch;
     size_t out_z_stride;
-    size_t lds_bytes() const { return 0; }
+    using Warp = WarpOfPixels<Sender>;
+    static constexpr bool WARPS_TILES = Warp::value && STREAMS_ROWS;
+    unsigned tile_dwords; // WARPS_TILES: the pixels of a source box that a block can hold, if the output is cut into tiles (warp_tile), or 0
+    size_t lds_bytes() const { return tile_dwords != 0u ? (tile_dwords + 4u) * 4u : 0u; }
+    // A warp's tiles, decided by the host: enough of them to fill the chip, slanted ones, and source boxes that fit the LDS (looked up
+    // at the output's corners and centre; a block whose own box does not fit takes its taps from memory).
+    unsigned plan_tiles() {
+        if constexpr (WARPS_TILES) {
+            const unsigned gx = (active.x + WARP_TILE_W - 1u) / WARP_TILE_W, gy = (active.y + WARP_TILE_H - 1u) / WARP_TILE_H;
+            const auto& src = sender.backIOp.params;
+            if (active.z != 1u || static_cast<size_t>(gx) * gy < WARP_MIN_BLOCKS || gy > 65535u) return 0u;
+            if (SourceAccess<PlainView<typename Warp::Pixel>>::quad_extent(Warp::view(src)) >= (size_t(1) << 31)) return 0u;
+            float largest = 0.f;
+            bool slanted = false;
+            const int last_x = static_cast<int>(active.x) - WARP_TILE_W, last_y = static_cast<int>(active.y) - WARP_TILE_H;
+            for (int at = 0; at < 5; ++at) {
+                const int x0 = at == 4 ? last_x / 2 : (at & 1) != 0 ? last_x : 0, y0 = at == 4 ? last_y / 2 : (at & 2) != 0 ? last_y : 0;
+                float lo_x = 0.f, hi_x = 0.f, lo_y = 0.f, hi_y = 0.f;
+                for (int c = 0; c < 4; ++c) {
+                    const float2 p = Warp::Coords::exec(Point(x0 + (c & 1) * (WARP_TILE_W - 1), y0 + (c >> 1) * (WARP_TILE_H - 1)), sender.params);
+                    lo_x = c == 0 || p.x < lo_x ? p.x : lo_x;
+                    hi_x = c == 0 || p.x > hi_x ? p.x : hi_x;
+                    lo_y = c == 0 || p.y < lo_y ? p.y : lo_y;
+                    hi_y = c == 0 || p.y > hi_y ? p.y : hi_y;
+                }
+                const float2 first = Warp::Coords::exec(Point(x0, y0), sender.params), last = Warp::Coords::exec(Point(x0 + WARP_TILE_W - 1, y0), sender.params);
+                const float crossed = last.y > first.y ? last.y - first.y : first.y - last.y;
+                slanted = slanted || crossed >= (Warp::TYPE == WarpType::Affine ? WARP_SLANT_AFFINE : WARP_SLANT_PERSPECTIVE);
+                const float box = (hi_x - lo_x + 9.f) * (hi_y - lo_y + 4.f);
+                if (!(box <= static_cast<float>(WARP_TILE_DWORDS))) return 0u; // (not for NaN either)
+                largest = box > largest ? box : largest;
+            }
+            if (!slanted) return 0u;
+            grid_x = gx;
+            grid_y = gy;
+            const unsigned room = static_cast<unsigned>(largest * 1.125f) + 64u; // (boxes between the five are a little larger at most)
+            return room < WARP_TILE_DWORDS ? room & ~3u : WARP_TILE_DWORDS;
+        } else {
+            return 0u;
+        }
+    }
     // decides the elements per thread from the size of the output and returns the number of blocks along x
     unsigned plan(const ActiveThreads& extent) {
         const size_t elems = static_cast<size_t>(extent.x) * extent.y * extent.z;
@@ -2095,10 +2168,139 @@ struct GenericJob {
             if (x0 + STEP * k < w) Receiver::Operation::exec(Point(x0 + STEP * k, y, static_cast<int>(bz)), value[k], job.receiver);
         }
     }
-    __device__ __attribute__((always_inline)) static inline void run(const GenericJob& job, unsigned bx, unsigned by, unsigned bz, unsigned char*) {
+    // One tile of a warp.  What one pixel computes is the operations' own code (coordinates, taps, blend) on the same values.
+    __device__ __attribute__((always_inline)) static inline void warp_tile(const GenericJob& job, const Held& held, unsigned bx, unsigned by, unsigned char* lds) {
+        using Pixel = typename Warp::Pixel;
+        using Access = SourceAccess<PlainView<Pixel>>;
+        const int tid = dev::thread_in_block();
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int lane = tid & 63;
+        const auto params = job.sender.params;
+        const auto src = job.sender.backIOp.params;
+        const int w = static_cast<int>(held.active.x), h = static_cast<int>(held.active.y);
+        const int src_w = static_cast<int>(src.dims.width), src_h = static_cast<int>(src.dims.height);
+        const int x0 = static_cast<int>(bx) * WARP_TILE_W, y0 = static_cast<int>(by) * WARP_TILE_H;
+        unsigned int* const tile = reinterpret_cast<unsigned int*>(lds);
+
+        // the box, from a corner per lane (the first of every four lanes speaks for all: each four hold the four corners)
+        const auto least = [](const int a, const int b) { return a < b ? a : b; };
+        const float2 corner = Warp::Coords::exec(Point((lane & 1) != 0 ? least(x0 + WARP_TILE_W - 1, w - 1) : x0, (lane & 2) != 0 ? least(y0 + WARP_TILE_H - 1, h - 1) : y0), params);
+        const auto over_corners = [](const float v, const auto pick) {
+            const auto swapped = [](const float f, const auto control) {
+                return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, f), decltype(control)::value, 0xf, 0xf, true));
+            };
+            float m = pick(v, swapped(v, std::integral_constant<int, 0xB1>{})); // lanes 1 0 3 2
+            m = pick(m, swapped(m, std::integral_constant<int, 0x4E>{}));       // lanes 2 3 0 1
+            return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
+        };
+        const auto lower = [](const float a, const float b) { return __builtin_fminf(a, b); };
+        const auto higher = [](const float a, const float b) { return __builtin_fmaxf(a, b); };
+        // (clamped as floats, so that the conversion is of a value inside the image also where a corner is infinite or no number)
+        const auto clamped = [](const float v, const int size) {
+            return __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_floorf(__builtin_fminf(__builtin_fmaxf(v, 0.f), static_cast<float>(size - 1)))));
+        };
+        const int q_lo = clamped(over_corners(corner.x, lower) - WARP_BOX_MARGIN, src_w) >> 2;
+        const int quads = (clamped(over_corners(corner.x, higher) + (1.f + WARP_BOX_MARGIN), src_w) >> 2) - q_lo + 1;
+        const int r_lo = clamped(over_corners(corner.y, lower) - WARP_BOX_MARGIN, src_h);
+        const int rows = clamped(over_corners(corner.y, higher) + (1.f + WARP_BOX_MARGIN), src_h) - r_lo + 1;
+        const int items = quads * rows;
+        const bool staged = quads > 0 && rows > 0 && quads <= 127 && static_cast<unsigned>(items) * 4u <= job.tile_dwords; // (uniform)
+        if (staged) {
+            const PlainView<Pixel> view{ src.data, src.dims.pitch, src_w, src_h, 0, 0, src_w, src_h };
+            const __amdgpu_buffer_rsrc_t image = Access::quad_buffer(view);
+            // item / quads by a multiplication: exact for the items of a box that fits (at most 2048, rows of at most 127 groups)
+            const unsigned m = static_cast<unsigned>(1048576.0f * __builtin_amdgcn_rcpf(static_cast<float>(quads))) + 2u;
+            const auto fill = [&](const auto any) {
+                constexpr bool ANY = decltype(any)::value;
+                constexpr int PASSES = 2;
+                for (int first = 0; first < items; first += BLOCK_THREADS * PASSES) { // (uniform)
+                    typename Access::template RawQuad<ANY> raw[PASSES];
+#pragma unroll
+                    for (int u = 0; u < PASSES; ++u) { // (no branch between the loads: groups past the last repeat it, from the cache)
+                        const int wanted = first + BLOCK_THREADS * u + tid;
+                        const int item = wanted < items ? wanted : items - 1;
+                        const int r = static_cast<int>((static_cast<unsigned>(item) * m) >> 20);
+                        Access::template load_quad<ANY>(image, view, q_lo + (item - r * quads), r_lo + r, raw[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < PASSES; ++u) {
+                        if (first + BLOCK_THREADS * u + 64 * wave < items) { // (uniform: some group of this wave's pass exists)
+                            const int wanted = first + BLOCK_THREADS * u + tid;
+                            const int item = wanted < items ? wanted : items - 1;
+                            unsigned int px[4];
+                            Access::template quad_dwords<ANY>(raw[u], px);
+                            dev::u32x4 piece;
+                            piece.x = px[0]; piece.y = px[1]; piece.z = px[2]; piece.w = px[3];
+                            *reinterpret_cast<dev::u32x4*>(tile + item * 4) = piece;
+                        }
+                    }
+                }
+            };
+            if (Access::quads_aligned(view)) fill(std::false_type{});
+            else fill(std::true_type{});
+        }
+        dev::block_sync();
+        // (columns and rows past the output's last repeat it)
+        const int x = least(x0 + lane, w - 1);
+        const bool column_here = x0 + lane < w;
+        const int wave_y = y0 + wave * WARP_ROWS;
+        if (staged) {
+            const int c_lo = q_lo * 4, stride = quads * 4;
+            // tap columns and rows whose right and lower neighbours are in the tile, or are themselves (the image's last)
+            const unsigned taps_x = static_cast<unsigned>(c_lo + stride >= src_w ? src_w - c_lo : stride - 1);
+            const unsigned taps_y = static_cast<unsigned>(r_lo + rows >= src_h ? src_h - r_lo : rows - 1);
+            Value value[WARP_ROWS];
+            unsigned long long missed = 0ull;
+#pragma unroll
+            for (int k = 0; k < WARP_ROWS; ++k) {
+                const float2 at = Warp::Coords::exec(Point(x, least(wave_y + k, h - 1)), params);
+                const bool inside = at.x >= 0.f && at.x < src_w && at.y >= 0.f && at.y < src_h;
+                const fk::detail::BilinearTaps t = fk::detail::bilinear_taps(at.x, at.y, Size(src_w, src_h));
+                const unsigned cx = static_cast<unsigned>(t.x1 - c_lo), cy = static_cast<unsigned>(t.y1 - r_lo);
+                const bool in_tile = inside && cx < taps_x && cy < taps_y;
+                missed |= __builtin_amdgcn_ballot_w64(inside && !in_tile);
+                const unsigned up = in_tile ? (cy & 2047u) * (static_cast<unsigned>(stride) & 511u) + cx : 0u;
+                const unsigned down = up + (in_tile && t.y2r != t.y1 ? static_cast<unsigned>(stride) : 0u);
+                const unsigned int a = tile[up], c = tile[down];
+                unsigned int b = tile[up + 1u], d = tile[down + 1u];
+                b = t.x2r != t.x1 ? b : a;
+                d = t.x2r != t.x1 ? d : c;
+                const Value sample = fk::detail::bilinear_blend(dev::unpack3<Pixel>(a), dev::unpack3<Pixel>(b), dev::unpack3<Pixel>(c), dev::unpack3<Pixel>(d), t);
+                value[k] = inside ? sample : make_set<Value>(0.f);
+            }
+            if (missed == 0ull) { // (uniform)
+                if (held.stream_rows != 0u) {
+                    const __amdgpu_buffer_rsrc_t rows_buffer = dev::wave_buffer(dev::wave_uniform(held.out_data + static_cast<size_t>(wave_y) * held.out_pitch));
+#pragma unroll
+                    for (int k = 0; k < WARP_ROWS; ++k) {
+                        if (column_here && wave_y + k < h) {
+                            dev::stream_store_at<dev::WordsOf<Value>::ND>(rows_buffer, static_cast<unsigned>(x) * static_cast<unsigned>(sizeof(Value)), static_cast<unsigned>(k) * held.out_pitch,
+                                                                          dev::WordsOf<Value>::of(value[k]));
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < WARP_ROWS; ++k) {
+                        if (column_here && wave_y + k < h) Receiver::Operation::exec(Point(x, wave_y + k, 0), value[k], job.receiver);
+                    }
+                }
+                return;
+            }
+        }
+        for (int k = 0; k < WARP_ROWS; ++k) {
+            if (column_here && wave_y + k < h) Receiver::Operation::exec(Point(x, wave_y + k, 0), Sender::Operation::exec(Point(x, wave_y + k, 0), job.sender), job.receiver);
+        }
+    }
+    __device__ __attribute__((always_inline)) static inline void run(const GenericJob& job, unsigned bx, unsigned by, unsigned bz, unsigned char* lds) {
         const Held held{ job.active, job.stream_rows, job.packs_rows, job.out_data, job.out_pitch, job.out_z_stride };
         const unsigned wide = job.wide, bands = job.xcd_bands, gx = job.grid_x, gy = job.grid_y;
         if (bands != 0u) dev::xcd_band_block(bx, by, bz, gx, gy, held.active.z);
+        if constexpr (WARPS_TILES) {
+            if (job.tile_dwords != 0u) {
+                warp_tile(job, held, bx, by, lds);
+                return;
+            }
+        }
         if constexpr (PACKS_ROWS) { // the only jobs that are compiled with the neighbour form
             if (wide != 0u && held.packs_rows != 0u) {
                 body<4, true>(job, held, bx, by, bz);

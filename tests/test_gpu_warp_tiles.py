@@ -1,0 +1,56 @@
+"""Warps whose outputs are cut into tiles (1024 tiles of 64 x 16 and more, slanted): source boxes from LDS, at every alignment of the
+source's rows, and the blocks of such a launch that take their taps from memory (boxes too large, coordinates that the corners
+do not bound); against the CPU oracle, bit for bit."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import same_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def at_byte(img, start, extra):
+    """`img` (h, w, 3) in device memory, its first pixel `start` bytes behind a dword, rows `extra` bytes further apart than tight."""
+    h, w, _ = img.shape
+    pitch = 3 * w + extra
+    flat = np.full(start + h * pitch, 170, np.uint8)
+    flat[start:].reshape(h, pitch)[:, :3 * w] = img.reshape(h, 3 * w)
+    return torch.as_strided(torch.from_numpy(flat).cuda(), (h, w, 3), (pitch, 3, 1), start)
+
+
+def rotation(degrees, scale, src, dst):
+    a = math.radians(degrees)
+    c, s = scale * math.cos(a), scale * math.sin(a)
+    return [[c, -s, src[0] / 2 - c * dst[0] / 2 + s * dst[1] / 2], [s, c, src[1] / 2 - s * dst[0] / 2 - c * dst[1] / 2]]
+
+
+AFFINE = [(0, 1), (3.5, 1), (5, 1), (-20, 0.5), (45, 1.3), (90, 1), (180, 1), (10, 1.9), (30, 3)]
+
+
+# widths around a tile's, outputs with and without streaming stores (4 MiB), tall and narrow ones
+@pytest.mark.parametrize("src,start,extra,dst", [((1021, 700), 0, 0, (1100, 1000)), ((1022, 701), 1, 0, (1025, 1009)), ((1024, 640), 0, 0, (2048, 512)),
+                                                 ((999, 333), 3, 2, (129, 5462)), ((64, 48), 0, 0, (1088, 1024)), ((1, 1), 2, 0, (1088, 1024)), ((3, 777), 0, 4, (1088, 1024))])
+def test_affine_tiles(fk, oracle, src, start, extra, dst):
+    img = oracle.bytes(70 + src[0], (src[1], src[0], 3))
+    d_src = at_byte(img, start, extra)
+    for degrees, scale in AFFINE:
+        m = rotation(degrees, scale, src, dst)
+        out = torch.full((dst[1], dst[0], 3), float("nan"), device="cuda")
+        fk.warp_u8c3_f32c3(fk.WARP_AFFINE, m, d_src, out)
+        assert same_bits(out.cpu().numpy(), oracle.warp_u8c3_f32c3(fk.WARP_AFFINE, m, img, dst)), (degrees, scale)
+
+
+# a slight tilt; a horizon that crosses the output; a scale that grows across it until boxes no longer fit
+@pytest.mark.parametrize("third", [[4e-5, 2e-5, 1.0], [-1.2e-3, 1e-4, 1.0], [-8e-4, -1e-4, 1.0], [0.0, 0.0, 0.0], [float("inf"), 0.0, 1.0]])
+def test_perspective_tiles(fk, oracle, third):
+    src, dst = (1023, 767), (1090, 1030)
+    img = oracle.bytes(91, (src[1], src[0], 3))
+    d_src = at_byte(img, 1, 1)
+    for rows in (rotation(14, 0.9, src, dst), rotation(-40, 0.6, src, dst), [[0.5, 0.0, 3.0], [0.3, 0.5, -40.0]]):
+        m = rows + [third]
+        out = torch.full((dst[1], dst[0], 3), float("nan"), device="cuda")
+        fk.warp_u8c3_f32c3(fk.WARP_PERSPECTIVE, m, d_src, out)
+        assert same_bits(out.cpu().numpy(), oracle.warp_u8c3_f32c3(fk.WARP_PERSPECTIVE, m, img, dst))
