@@ -54,18 +54,25 @@ void require(const bool condition, const char* text) {
 }
 
 // ---- Python values -------------------------------------------------------------------------------------------------------
+int low_bits(PyObject* integer) { // as a C int takes them, without a range check
+    const unsigned long v = PyLong_AsUnsignedLongMask(integer);
+    if (v == static_cast<unsigned long>(-1) && PyErr_Occurred()) throw PythonError{};
+    return static_cast<int>(v);
+}
+int to_index(PyObject* o) { // whole numbers only: a float or a text is refused
+    PyObject* const n = PyNumber_Index(o);
+    if (n == nullptr) throw PythonError{};
+    const int v = low_bits(n);
+    Py_DECREF(n);
+    return v;
+}
 int to_int(PyObject* o) { // int(o)
-    if (PyLong_Check(o)) {
-        const long v = PyLong_AsLong(o);
-        if (v == -1 && PyErr_Occurred()) throw PythonError{};
-        return static_cast<int>(v);
-    }
+    if (PyLong_Check(o)) return low_bits(o);
     PyObject* const n = PyNumber_Long(o);
     if (n == nullptr) throw PythonError{};
-    const long v = PyLong_AsLong(n);
+    const int v = low_bits(n);
     Py_DECREF(n);
-    if (v == -1 && PyErr_Occurred()) throw PythonError{};
-    return static_cast<int>(v);
+    return v;
 }
 float to_float(PyObject* o) {
     const double v = PyFloat_AsDouble(o);
@@ -108,18 +115,18 @@ Byte3 to_byte3(PyObject* o) {
     for (int i = 0; i < v.size(); ++i) b[static_cast<size_t>(i)] = static_cast<uint8_t>(to_int(v[i]));
     return b;
 }
-fk_rect to_rect(PyObject* o) {
+fk_rect to_rect(PyObject* o, int (*value)(PyObject*)) { // value: to_int, or to_index where a region is of whole numbers only
     const Items v(o);
     if (v.size() > 4) raise(PyExc_TypeError, "a region is (x, y, width, height)");
     int f[4] = { 0, 0, 0, 0 };
-    for (int i = 0; i < v.size(); ++i) f[i] = to_int(v[i]);
+    for (int i = 0; i < v.size(); ++i) f[i] = value(v[i]);
     return fk_rect{ f[0], f[1], f[2], f[3] };
 }
 std::vector<fk_rect> to_rects(PyObject* o) {
     const Items v(o);
     std::vector<fk_rect> r;
     r.reserve(static_cast<size_t>(v.size()));
-    for (int i = 0; i < v.size(); ++i) r.push_back(to_rect(v[i]));
+    for (int i = 0; i < v.size(); ++i) r.push_back(to_rect(v[i], to_int));
     return r;
 }
 void* to_stream(PyObject* o) {
@@ -253,7 +260,7 @@ PyObject* readme(Args a, decltype(&::fk_crop_resize_muls_bgr_tensor) fn) { // sr
     const Planes o = packed_planes(a[2]);
     const std::vector<fk_rect> rects = to_rects(a[1]);
     require(o.n == static_cast<int>(rects.size()), "one plane of the result per region");
-    const int aspect = to_int(a[3]);
+    const int aspect = to_index(a[3]);
     const Float3 bg = to_float3(a[4]), mul = to_float3(a[5]), sub = to_float3(a[6]), div = to_float3(a[7]);
     void* const stream = to_stream(a[8]);
     return now_or_deferred(a[9], a[2], [=] {
@@ -266,7 +273,7 @@ PyObject* crop_resize_muls_bgr_tensor_noalloc(Args a) { return readme(a, lib.fk_
 PyObject* muladd_chain_f32c3(Args a) { // src, dst, depth, mul_v, add_v, stream, defer
     const ImageArg s = image(floats(a[0])), d = image(floats(a[1]));
     require(s.w == d.w && s.h == d.h, "images of one size");
-    const int depth = to_int(a[2]);
+    const int depth = to_index(a[2]);
     const float mul = to_float(a[3]), add = to_float(a[4]);
     void* const stream = to_stream(a[5]);
     return now_or_deferred(a[6], a[1], [=, fn = lib.fk_muladd_chain_f32c3] { return fn(s.data, s.w, s.h, s.pitch, depth, mul, add, d.data, d.pitch, stream); });
@@ -301,7 +308,7 @@ PyObject* resize_crop_tiles(Args a) { // src, resized, rects, out, mul, stream, 
     require(o.n == static_cast<int>(rects.size()), "one plane of the result per tile");
     const Items resized(a[1]);
     if (resized.size() < 2) raise(PyExc_IndexError, "resized is (width, height)");
-    const int rw = to_int(resized[0]), rh = to_int(resized[1]);
+    const int rw = to_index(resized[0]), rh = to_index(resized[1]);
     const Float3 mul = to_float3(a[4]);
     void* const stream = to_stream(a[5]);
     return now_or_deferred(a[6], a[3], [=, fn = lib.fk_resize_crop_tiles] { return fn(s.data, s.w, s.h, s.pitch, rw, rh, rects.data(), o.n, o.w, o.h, mul.data(), o.data, stream); });
@@ -322,8 +329,8 @@ PyObject* resize_mul_u8c4_f32c4(Args a) { // src, dst, mul_v, stream, defer
 }
 PyObject* crop_mul_saturate_u8c4(Args a) { // src, rect, dst, mul_v, stream, defer
     const ImageArg s = image(bytes(a[0])), d = image(bytes(a[2]));
-    const fk_rect r = to_rect(a[1]);
-    const int mul = to_int(a[3]);
+    const fk_rect r = to_rect(a[1], to_index);
+    const int mul = to_index(a[3]);
     void* const stream = to_stream(a[4]);
     return now_or_deferred(a[5], a[2], [=, fn = lib.fk_crop_mul_saturate_u8c4] { return fn(s.data, s.w, s.h, s.pitch, r, mul, d.data, d.pitch, stream); });
 }
@@ -339,8 +346,8 @@ PyObject* divergent4_u8c4(Args a) { // src, gray_out, resized_out, mul_b, rect_c
     void* const gray = bytes(a[1]).data_ptr();
     const ImageArg resized = image(floats(a[2]));
     const float mul_b = to_float(a[3]), sub_d = to_float(a[7]);
-    const fk_rect r = to_rect(a[4]);
-    const int mul_c = to_int(a[5]);
+    const fk_rect r = to_rect(a[4], to_index);
+    const int mul_c = to_index(a[5]);
     void* const crop = bytes(a[6]).data_ptr();
     void* const bgr = floats(a[8]).data_ptr();
     void* const stream = to_stream(a[9]);
@@ -372,21 +379,21 @@ PyObject* batch_windows_saturate_muls_f32(Args a) { // src, rects, out, mul_v, s
 }
 
 PyObject* read_yuv(Args a) { // fmt, raw, out, stream, defer
-    const int fmt = to_int(a[0]);
+    const int fmt = to_index(a[0]);
     const RawArg raw = raw_image(a[1], fmt);
     const ImageArg o = image(pixels(a[2]));
     void* const stream = to_stream(a[3]);
     return now_or_deferred(a[4], a[2], [=, fn = lib.fk_read_yuv] { return fn(fmt, raw.data, raw.pitch, o.w, o.h, o.data, o.pitch, stream); });
 }
 PyObject* write_yuv(Args a) { // fmt, pixels, raw, stream, defer
-    const int fmt = to_int(a[0]);
+    const int fmt = to_index(a[0]);
     const ImageArg p = image(pixels(a[1]));
     const RawArg raw = raw_image(a[2], fmt);
     void* const stream = to_stream(a[3]);
     return now_or_deferred(a[4], a[2], [=, fn = lib.fk_write_yuv] { return fn(fmt, p.data, p.pitch, p.w, p.h, raw.data, raw.pitch, stream); });
 }
 PyObject* yuv_to_rgb(Args a) { // fmt, color_range, primaries, raw, out, stream, defer
-    const int fmt = to_int(a[0]), range = to_int(a[1]), primaries = to_int(a[2]);
+    const int fmt = to_index(a[0]), range = to_index(a[1]), primaries = to_index(a[2]);
     const RawArg raw = raw_image(a[3], fmt);
     const at::Tensor& out = pixels(a[4]);
     const ImageArg o = image(out);
@@ -397,12 +404,12 @@ PyObject* yuv_to_rgb(Args a) { // fmt, color_range, primaries, raw, out, stream,
     return now_or_deferred(a[6], a[4], [=, fn = lib.fk_yuv_to_rgb] { return fn(fmt, range, primaries, alpha, float_out, raw.data, raw.pitch, o.w, o.h, o.data, o.pitch, stream); });
 }
 PyObject* yuv_crop_resize_norm_split(Args a) { // fmt, color_range, primaries, raw, size, crop, out, div_v, stream, defer
-    const int fmt = to_int(a[0]), range = to_int(a[1]), primaries = to_int(a[2]);
+    const int fmt = to_index(a[0]), range = to_index(a[1]), primaries = to_index(a[2]);
     const RawArg raw = raw_image(a[3], fmt);
     const Items size(a[4]);
     if (size.size() < 2) raise(PyExc_IndexError, "size is (width, height)");
-    const int w = to_int(size[0]), h = to_int(size[1]);
-    const fk_rect crop = to_rect(a[5]);
+    const int w = to_index(size[0]), h = to_index(size[1]);
+    const fk_rect crop = to_rect(a[5], to_int);
     const at::Tensor& out = floats(a[6]);
     if (out.dim() != 3) raise(PyExc_ValueError, "out is (3, height, width)");
     require(out.is_contiguous(), "the result must be contiguous");
@@ -414,14 +421,14 @@ PyObject* yuv_crop_resize_norm_split(Args a) { // fmt, color_range, primaries, r
 }
 
 PyObject* border_crop_u8c3(Args a) { // border_type, src, left, top, out, value, stream, defer
-    const int type = to_int(a[0]), left = to_int(a[2]), top = to_int(a[3]);
+    const int type = to_index(a[0]), left = to_int(a[2]), top = to_int(a[3]);
     const ImageArg s = image(bytes(a[1])), o = image(bytes(a[4]));
     const Byte3 value = to_byte3(a[5]);
     void* const stream = to_stream(a[6]);
     return now_or_deferred(a[7], a[4], [=, fn = lib.fk_border_crop_u8c3] { return fn(type, s.data, s.w, s.h, s.pitch, left, top, o.w, o.h, value.data(), o.data, o.pitch, stream); });
 }
 PyObject* warp_u8c3_f32c3(Args a) { // warp_type, matrix, src, out, stream, defer
-    const int type = to_int(a[0]);
+    const int type = to_index(a[0]);
     const ImageArg s = image(bytes(a[2])), o = image(floats(a[3]));
     std::array<float, 9> m{}; // row-major, given flat or as rows
     int given = 0;
@@ -443,7 +450,7 @@ PyObject* warp_u8c3_f32c3(Args a) { // warp_type, matrix, src, out, stream, defe
     return now_or_deferred(a[5], a[3], [=, fn = lib.fk_warp_u8c3_f32c3] { return fn(type, m.data(), s.data, s.w, s.h, s.pitch, o.w, o.h, o.data, o.pitch, stream); });
 }
 PyObject* deinterlace_u8c3_f32c3(Args a) { // kind, use_even_lines, src, out, stream, defer
-    const int kind = to_int(a[0]), even = to_int(a[1]);
+    const int kind = to_index(a[0]), even = to_int(a[1]);
     const ImageArg s = image(bytes(a[2])), o = image(floats(a[3]));
     require(s.w == o.w && s.h == o.h, "images of one size");
     void* const stream = to_stream(a[4]);
@@ -451,7 +458,7 @@ PyObject* deinterlace_u8c3_f32c3(Args a) { // kind, use_even_lines, src, out, st
 }
 
 PyObject* tensor_relayout_f32c3(Args a) { // mode, src, w, h, planes, out, stream, defer
-    const int mode = to_int(a[0]), w = to_int(a[2]), h = to_int(a[3]), planes = to_int(a[4]);
+    const int mode = to_index(a[0]), w = to_index(a[2]), h = to_index(a[3]), planes = to_index(a[4]);
     const at::Tensor &src = floats(a[1]), &out = floats(a[5]);
     require(src.is_contiguous() && out.is_contiguous() && src.numel() == out.numel() && src.numel() == static_cast<int64_t>(planes) * h * w * 3, "contiguous tensors of planes * h * w * 3 elements");
     const float* const s = static_cast<const float*>(src.data_ptr());
@@ -460,7 +467,7 @@ PyObject* tensor_relayout_f32c3(Args a) { // mode, src, w, h, planes, out, strea
     return now_or_deferred(a[7], a[5], [=, fn = lib.fk_tensor_relayout_f32c3] { return fn(mode, s, w, h, planes, o, stream); });
 }
 PyObject* circular_tensor_read_f32c3(Args a) { // direction, first, ring, out, stream, defer
-    const int direction = to_int(a[0]), first = to_int(a[1]);
+    const int direction = to_index(a[0]), first = to_index(a[1]);
     const Planes r = packed_planes(a[2]), o = packed_planes(a[3]);
     require(to_tensor(a[2]).sizes() == to_tensor(a[3]).sizes(), "tensors of one shape");
     void* const stream = to_stream(a[4]);
@@ -472,7 +479,7 @@ PyObject* circular_tensor_update_u8c3_split_f32(Args a) { // frame, mul_v, tenso
     const at::Tensor &tensor = floats(a[2]), &ring = floats(a[3]);
     const auto fits = [&](const at::Tensor& t) { return t.dim() == 4 && t.is_contiguous() && t.size(0) == tensor.size(0) && t.size(1) == 3 && t.size(2) == f.h && t.size(3) == f.w; };
     require(fits(tensor) && fits(ring), "tensor and ring are (batch, 3, h, w), contiguous");
-    const int batch = static_cast<int>(tensor.size(0)), next = to_int(a[4]), newest = to_int(a[5]);
+    const int batch = static_cast<int>(tensor.size(0)), next = to_index(a[4]), newest = to_int(a[5]);
     float *const t = static_cast<float*>(tensor.data_ptr()), *const r = static_cast<float*>(ring.data_ptr());
     void* const stream = to_stream(a[6]);
     PyObject* const done = now_or_deferred(a[7], Py_None, [=, fn = lib.fk_circular_tensor_update_u8c3_split_f32] { return fn(f.data, f.w, f.h, f.pitch, mul, t, r, batch, next, newest, stream); });

@@ -113,3 +113,22 @@ def test_refusals(fk, case):
     bound = fk.crop_resize_muls_bgr_tensor(src, [(0, 0, 400, 20)] * 5, out, *VALUES, defer=True)
     with pytest.raises(fk.FkError, match="outside"):
         bound()
+
+
+def test_whole_numbers(fk, case):
+    """Kinds, counts and sizes are whole numbers: a float that only a conversion would make one is refused, integers of any type are taken."""
+    src, want = case
+    out = torch.empty((5, 60, 60, 3), device="cuda")
+    rgba, crop = torch.zeros((32, 48, 4), dtype=torch.uint8, device="cuda"), torch.empty((8, 8, 4), dtype=torch.uint8, device="cuda")
+    floats, raw = torch.zeros((16, 16, 3), device="cuda"), torch.zeros((24, 16), dtype=torch.uint8, device="cuda")
+    yuv, planes = torch.empty((16, 16, 3), dtype=torch.uint8, device="cuda"), torch.empty((3, 8, 8), device="cuda")
+    for call in [lambda: fk.crop_resize_muls_bgr_tensor(src, RECTS, out, 0.0, *VALUES[1:]), lambda: fk.crop_resize_muls_bgr_tensor(src, RECTS, out, "0", *VALUES[1:]),
+                 lambda: fk.muladd_chain_f32c3(floats, floats, 4.0, 1.0, 0.0), lambda: fk.resize_crop_tiles(src, (80.0, 64), RECTS, out, (1.0,) * 3),
+                 lambda: fk.crop_mul_saturate_u8c4(rgba, (0, 0, 8, 8), crop, 2.0), lambda: fk.crop_mul_saturate_u8c4(rgba, (0.0, 0, 8, 8), crop, 2),
+                 lambda: fk.read_yuv(float(fk.NV12), raw, yuv), lambda: fk.warp_u8c3_f32c3(0.0, [1, 0, 0, 0, 1, 0], src, floats),
+                 lambda: fk.yuv_crop_resize_norm_split(fk.NV12, 0, 0, raw, (16.0, 16), (0, 0, 8, 8), planes, 255.0)]:
+        with pytest.raises(TypeError):
+            call()
+    fk.crop_resize_muls_bgr_tensor(src, RECTS, out, torch.tensor(VALUES[0]), *VALUES[1:])
+    assert same_bits(out.cpu().numpy(), want)
+    fk.crop_mul_saturate_u8c4(rgba, tuple(np.array((0, 0, 8, 8))), crop, np.int32(2))
